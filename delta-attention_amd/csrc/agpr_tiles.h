@@ -1,9 +1,10 @@
-// O accumulator tiles of the 64-rows-per-wave attention kernels, held in
-// AGPRs a[128:255] outside the compiler's register allocation: tile i is
-// a[128 + 16 i : 143 + 16 i]. Every statement here names the registers it
-// touches as clobbers, so the compiler keeps no value of its own in them
-// across these statements; that it places none there at all is checked on
-// the kernels' assembly by tests/test_agpr_reserve.py.
+// O accumulator tiles of the one-wave-per-SIMD attention kernels (64 rows per
+// wave, and head_dim 256), held in AGPRs a[128:255] outside the compiler's
+// register allocation: tile i is a[128 + 16 i : 143 + 16 i]. Every statement
+// here names the registers it touches as clobbers, so the compiler keeps no
+// value of its own in them across these statements; that it places none there
+// at all is checked on the kernels' assembly by tests/test_agpr_reserve.py and
+// tests/test_agpr_reserve_d256.py.
 //
 // Hazards (the compiler pads only the MFMAs it emits itself):
 //  * an 8-pass XDL MFMA's result needs NumPasses + 3 wait states before a

@@ -17,7 +17,8 @@
 //     (64 rows per wave, BM = 256, one workgroup and one wave per SIMD per CU):
 //     every K and V fragment read from LDS feeds one MFMA per row group, half
 //     the LDS bytes per MFMA of RG = 1 (32 rows per wave, BM = 128, two
-//     workgroups per CU), which the other head dims and the decode rows use.
+//     workgroups per CU), which the other head dims and the decode rows use
+//     (one workgroup per CU at head_dim 256).
 //   * Scores are formed transposed, S^T = K * Q^T, with v_mfma_f32_32x32x16
 //     (A = 32 keys x 16 dims from LDS, B = Q^T fragment kept in registers). In
 //     the 32x32 accumulator layout a lane holds one query row (lane % 32) of
@@ -225,6 +226,12 @@ __device__ __forceinline__ void wait_vmcnt() {
 // Workgroups per CU: two at 32 rows per wave and head_dim <= 128; one at 64
 // rows per wave (a wave's accumulators, scores and Q fragments take most of a
 // SIMD's 512 registers) and at head_dim 256 (whose K/V stages take 128 KB).
+// The one-wave-per-SIMD kernels run the static schedule of `step`, with O and
+// the Q fragments in AGPRs. For head_dim 256 it replaced the compiler's own
+// order, which kept O in the VGPRs and moved scores and fragments through
+// AGPRs on every tile (186 v_accvgpr_read per loop body): 509 rows of 16 heads
+// against 16901 keys 318 -> 212 us, 437 -> 655 TF/s (about 1.5 us per 64-key
+// tile, of which the DMAs cost 0.3; bound by its MFMA issue order).
 constexpr int attn_occupancy(int D, int RG) { return (D > 128 || RG > 1) ? 1 : 2; }
 
 template <typename T, int D, int MODE, int RG>
@@ -239,10 +246,11 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
   constexpr int NDMA = TL::BYTES / (NTHR * 16);   // 16-byte DMA chunks per thread per K (or V) tile
   constexpr float THRESH = Rescale<T>::thresh;
   constexpr float LSUM = Rescale<T>::lsum;
-  // 64 rows per wave: O lives in the reserved AGPR tiles of agpr_tiles.h
-  // (tile NDT * rg + dt), accumulated, scaled and read by asm only; the score
-  // MFMAs, whose results the softmax reads, stay compiler-built in VGPRs
-  constexpr bool AGPR_O = RG > 1;
+  // One wave per SIMD (64 rows per wave, or head_dim 256): O lives in the
+  // reserved AGPR tiles of agpr_tiles.h (tile NDT * rg + dt), accumulated,
+  // scaled and read by asm only; the score MFMAs, whose results the softmax
+  // reads, stay compiler-built in VGPRs
+  constexpr bool AGPR_O = attn_occupancy(D, RG) == 1;
   static_assert(!AGPR_O || RG * NDT <= 8, "eight reserved accumulator tiles");
   using E = Elt<T>;
 
@@ -355,15 +363,20 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
       const char* qp = (const char*)a.q + ((int64_t)b * a.qs_b + (int64_t)hrow[rg] * a.qs_h +
                                            (int64_t)qrow[rg] * a.qs_s) * esz;
 #pragma unroll
-      for (int ds = 0; ds < NDS; ++ds)
-        qf[rg][ds] = valid[rg] ? *(const u32x4*)(qp + (16 * ds + 8 * lg) * esz) : (u32x4){0, 0, 0, 0};
+      for (int ds = 0; ds < NDS; ++ds) {
+        // one wave per SIMD: no branch per load (each one waited for its load
+        // before the next, and no other wave covers that latency); a lane
+        // past the rows reads row 0 of the launch, and nothing of it is kept
+        if constexpr (AGPR_O) qf[rg][ds] = *(const u32x4*)(qp + (16 * ds + 8 * lg) * esz);
+        else qf[rg][ds] = valid[rg] ? *(const u32x4*)(qp + (16 * ds + 8 * lg) * esz) : (u32x4){0, 0, 0, 0};
+      }
     }
   };
-  // 64 rows per wave: the Q fragments stay in AGPRs, from which the score
+  // One wave per SIMD: the Q fragments stay in AGPRs, from which the score
   // MFMAs read their B operand directly (the VGPRs hold the two score tiles,
   // the packed probabilities and the addressing)
   auto pin_q = [&]() __attribute__((always_inline)) {
-    if constexpr (RG > 1) {
+    if constexpr (AGPR_O) {
 #pragma unroll
       for (int rg = 0; rg < RG; ++rg)
 #pragma unroll
@@ -625,7 +638,7 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
     // the SIMD fills those phases instead of competing for issue while this
     // one's MFMAs are ready (kernel (1) 0.9-1.3 % faster; the query-sparse
     // mode measured neutral to slower and keeps one priority).
-    constexpr bool PRIO = KSPARSE && RG == 1;
+    constexpr bool PRIO = KSPARSE && !AGPR_O;
     if constexpr (PRIO) __builtin_amdgcn_s_setprio(1);
     const int P = t & 1;
     if (t + 2 < nt) issue_k(t + 2, P);
@@ -639,34 +652,36 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
       const u32x2 v1 = read_tr16(vs + vread[dt] + (16 * kk + 4) * RB);
       return (u32x4){v0[0], v0[1], v1[0], v1[1]};
     };
-    if constexpr (RG > 1) {
+    if constexpr (AGPR_O) {
       // One wave per SIMD: nothing else on the SIMD hides the softmax or the
       // latencies of its dependent chain (FMA -> exp -> pack -> dot2), so the
       // step is one static software-pipelined schedule of NSL = 64 slots, one
-      // MFMA each: slots 0..31 the score MFMAs of S(t+1) (K fragment s / 2,
-      // row group s % 2; none in the last step), slots 32..63 the PV MFMAs
-      // (fragment f = (s - 32) / 2 = NDT kk + dt, row group s % 2). The 64
+      // MFMA each: slots 0..31 the score MFMAs of S(t+1) (K fragment s / RG,
+      // row group s % RG; none in the last step), slots 32..63 the PV MFMAs
+      // (fragment f = (s - 32) / RG = NDT kk + dt, row group s % RG). The NE
       // score elements per lane of S(t), in the order the PV MFMAs consume
-      // their pairs (e = 2 p + i, pair p = 8 kk + 4 rg + jj), have their
-      // exponential in slot xs(e) = 54 e / 64, the FMA one slot earlier, the
+      // their pairs (e = 2 p + i, pair p = 4 RG kk + 4 rg + jj), have their
+      // exponential in slot xs(e) = 54 e / NE, the FMA one slot earlier, the
       // pack one slot after the pair's second exponential and the row-sum dot2
       // two slots after that; a pair is packed at least two slots before its
       // first PV MFMA (the asm MFMAs' 2 wait states after a VALU write). K
-      // and V fragment reads run two fragments (four slots) ahead. Scheduling
-      // barriers between slots keep this order.
-      constexpr int NSL = 64, XS = 54;
-      static_assert(NQK * RG == 32 && 2 * NH * NDT * RG == 32 && RG * NH * 16 == 64,
-                    "64 MFMA slots and 64 score elements per lane");
+      // and V fragment reads run four slots ahead. Scheduling barriers
+      // between slots keep this order.
+      constexpr int NSL = 64, XS = 54, NE = RG * NH * 16;
+      constexpr int AH = 4 / RG;         // fragments read ahead
+      constexpr int NQ = AH + 1;         // fragment registers of the ring
+      static_assert(NQK * RG == 32 && 2 * NH * NDT * RG == 32, "64 MFMA slots");
       // element e -> (rg, hf, index within the half)
-      auto erg = [](int e) constexpr { return ((e / 2) / 4) % 2; };
-      auto ehf = [](int e) constexpr { return ((e / 2) / 8) / 2; };
-      auto ej = [](int e) constexpr { return 2 * (4 * (((e / 2) / 8) % 2) + (e / 2) % 4) + e % 2; };
+      auto erg = [](int e) constexpr { return ((e / 2) / 4) % RG; };
+      auto ekk = [](int e) constexpr { return (e / 2) / (4 * RG); };
+      auto ehf = [ekk](int e) constexpr { return ekk(e) / 2; };
+      auto ej = [ekk](int e) constexpr { return 2 * (4 * (ekk(e) % 2) + (e / 2) % 4) + e % 2; };
       const DA_LDS char* ks = lds0 + (P ^ 1) * (2 * TL::BYTES);
       auto kfrag = [&](int q) __attribute__((always_inline)) -> u32x4 {
         return *(const DA_LDS u32x4*)(ks + kread[q / NH] + 32 * (q % NH) * RB);
       };
-      u32x4 kq[3], vq[3];
-      float fv[64], xv[64];
+      u32x4 kq[NQ], vq[NQ];
+      float fv[NE], xv[NE];
       if (!LAST) {
 #pragma unroll
         for (int rg = 0; rg < RG; ++rg)
@@ -677,40 +692,39 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
       }
       __builtin_amdgcn_sched_barrier(0);
       // first element whose exponential is in slot x (xs is monotonic)
-      auto e_lo = [](int x) constexpr { return (64 * x + XS - 1) / XS; };
+      auto e_lo = [](int x) constexpr { return (NE * x + XS - 1) / XS; };
       StaticFor<0, NSL + 1>::run([&](auto i_c) __attribute__((always_inline)) {
         constexpr int sl = decltype(i_c)::value - 1;
         // fragment reads for the MFMAs four slots on
-        if constexpr (sl >= -1 && sl <= 2 * (NQK - 1) - 4) {
+        if constexpr (sl == -1) {
           if (!LAST) {
-            if constexpr (sl == -1) {
-              kq[0] = kfrag(0);
-              kq[1] = kfrag(1);
-            } else if constexpr (sl % 2 == 0) {
-              kq[((sl + 4) / 2) % 3] = kfrag((sl + 4) / 2);
-            }
+#pragma unroll
+            for (int q = 0; q < AH; ++q) kq[q] = kfrag(q);
           }
         }
-        if constexpr (sl >= 28 && sl % 2 == 0 && (sl - 28) / 2 < 2 * NH * NDT) {
-          constexpr int f = (sl - 28) / 2;
-          vq[f % 3] = vfrag(f / NDT, f % NDT);
+        if constexpr (sl >= 0 && sl < 32 && sl % RG == 0 && sl / RG + AH < NQK) {
+          if (!LAST) kq[(sl / RG + AH) % NQ] = kfrag(sl / RG + AH);
+        }
+        if constexpr (sl >= 28 && sl < 60 && sl % RG == 0) {
+          constexpr int f = (sl - 28) / RG;
+          vq[f % NQ] = vfrag(f / NDT, f % NDT);
         }
         // this slot's MFMA
         if constexpr (sl >= 0 && sl < 32) {
           if (!LAST) {
-            constexpr int q = sl / 2, rg = sl % 2;
-            nxt[rg][q % NH] = E::mfma(kq[q % 3], qf[rg][q / NH], nxt[rg][q % NH]);
+            constexpr int q = sl / RG, rg = sl % RG;
+            nxt[rg][q % NH] = E::mfma(kq[q % NQ], qf[rg][q / NH], nxt[rg][q % NH]);
           }
         } else if constexpr (sl >= 32) {
-          constexpr int f = (sl - 32) / 2, rg = sl % 2, kk = f / NDT, dt = f % NDT;
+          constexpr int f = (sl - 32) / RG, rg = sl % RG, kk = f / NDT, dt = f % NDT;
           const u32x4 pf = {pk[rg][4 * kk], pk[rg][4 * kk + 1], pk[rg][4 * kk + 2],
                             pk[rg][4 * kk + 3]};
-          ot_mfma<T, NDT * rg + dt>(vq[f % 3], pf);
+          ot_mfma<T, NDT * rg + dt>(vq[f % NQ], pf);
         }
         // this slot's softmax work: FMAs of the elements exponentiated in the
         // next slot (slot -1 also those of slot 0), exponentials, packs of the
         // pairs completed in the previous slot, dot2s three slots after
-        constexpr int f0 = sl == -1 ? 0 : e_lo(sl + 1), f1 = sl + 2 <= XS ? e_lo(sl + 2) : 64;
+        constexpr int f0 = sl == -1 ? 0 : e_lo(sl + 1), f1 = sl + 2 <= XS ? e_lo(sl + 2) : NE;
 #pragma unroll
         for (int e = f0; e < f1; ++e) fv[e] = fmaf(cur[erg(e)][ehf(e)][ej(e)], c2, -m_i[erg(e)]);
         if constexpr (sl >= 0 && sl < XS) {
@@ -854,19 +868,13 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
       step(t, Last(), exact_tag, sa, sb);
     }
   };
-  if constexpr (D > 128) {
-    // one wave per SIMD: the exact pass only (the first pass's second loop
-    // copy would not fit beside the head_dim-256 state without spills)
-    run(std::true_type());
-  } else {
-    run(std::false_type());
-    // the barrier inside also orders the first pass's last LDS reads before
-    // the second pass refills the stages
-    bool big = false;
+  run(std::false_type());
+  // the barrier inside also orders the first pass's last LDS reads before
+  // the second pass refills the stages
+  bool big = false;
 #pragma unroll
-    for (int rg = 0; rg < RG; ++rg) big = big || (valid[rg] && !(l_i[rg] <= 0.5f * LSUM));
-    if (__syncthreads_or(big)) run(std::true_type());
-  }
+  for (int rg = 0; rg < RG; ++rg) big = big || (valid[rg] && !(l_i[rg] <= 0.5f * LSUM));
+  if (__syncthreads_or(big)) run(std::true_type());
 
   // ---- epilogue ----
   if constexpr (AGPR_O) {
