@@ -149,7 +149,12 @@ struct AttnArgs {
   // [0, n_rows]) are computed; the items of their row tiles are spread over
   // the XCDs in contiguous ranges and the other blocks exit at once
   const int* n_rows_dev;
-  uint32_t* part_o; // [item][ws_rows][D / 2]: element pairs of each row's O / l
+  // live launches: the split length of a plan for n_live rows grows with the
+  // live row tiles (live_chunk): bound of a list's tiles, resident workgroups
+  int vis, slots;
+  // [item][ws_rows][D]: each row's O / l, float when part_f32, else elements
+  void* part_o;
+  int part_f32;
   float* part_ml;   // [item][2][ws_rows]  (running max, row sum)
   int ws_rows;      // workspace rows per item: min(bm, n_rows * G) (a tile's valid rows)
   // MODE_FUSED: dense anchor rows [B, n_anchor, Hq, D] (strides batch, head,
@@ -215,6 +220,17 @@ __device__ __forceinline__ void tile_list(int hi_max, int lo_min, int sink, int&
   n_second = hi_max >= 0 ? max(0, hi_max / BN - second_t0 + 1) : 0;
 }
 
+// Key tiles per split item of a launch of `tiles` live row tiles, planned as
+// `chunk` for fewer: one round of the resident slots, up to 80 tiles (the
+// host's one-round rule). The adaptive stride's chunks have 64 anchors where
+// they start and up to 256 once the stride has fallen; at the 20-tile items of
+// 64 rows, 256 rows x 32 heads at 40K keys took four rounds and 32 partials a
+// row.
+__device__ __forceinline__ int live_chunk(int chunk, int tiles, int vis, int slots) {
+  const int per_tile = max(slots / max(tiles, 1), 1);
+  return max(chunk, min((vis + per_tile - 1) / per_tile, 80));
+}
+
 // s_waitcnt immediate (gfx9 encoding) that waits until at most `vm` vector
 // memory operations are outstanding; LDS and export counters are not waited on.
 template <int VM>
@@ -275,6 +291,7 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
   const bool live = !KSPARSE && a.n_rows_dev;
   int w;
   int mt, split = 0, bh, hs = 0;
+  int chunk = a.chunk;
   if (live) {
     // items of the live row tiles only: (bh, split, mt < mt_live), each XCD
     // a contiguous range of them (the row tiles of one split share its
@@ -282,6 +299,7 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
     const int n_live = min(max(*a.n_rows_dev, 0), a.n_rows);
     const int mt_live = (int)(((int64_t)n_live * a.G + BMK - 1) / BMK);
     const int total = a.B * a.Hkv * a.n_splits * mt_live;
+    chunk = live_chunk(chunk, a.B * a.Hkv * mt_live, a.vis, a.slots);
     const int per = (total + 7) >> 3;
     if (mt_live == 0 || (int)(blockIdx.x >> 3) >= per) return;
     w = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
@@ -435,7 +453,7 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
   tile_list(hi_max, lo_min, sink, n_first, second_t0, n_second);
   int nt = n_first + n_second, t_off = 0;
   if (!KSPARSE) {
-    const int chunk = a.n_kv_dev ? max(1, (int)fdiv(nt + a.n_splits - 1, a.fd_sp)) : a.chunk;
+    if (a.n_kv_dev) chunk = max(1, (int)fdiv(nt + a.n_splits - 1, a.fd_sp));
     t_off = split * chunk;
     if (t_off >= nt) return;   // past the list: the merge skips this split
     nt = min(chunk, nt - t_off);
@@ -479,6 +497,13 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
     for (int c = 0; c < NDMA; ++c)
       dma16(rk, (DA_LDS void*)(&smem[slot][0][(c * NWAVE + wave) * 1024]), koff[c]);
   };
+  // key tile t into the V buffer of stage 1 (free until V(1) is issued)
+  auto issue_ref = [&](int t) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t rk = tile_rsrc(kbase, kend, krow_b, t);
+#pragma unroll
+    for (int c = 0; c < NDMA; ++c)
+      dma16(rk, (DA_LDS void*)(&smem[1][1][(c * NWAVE + wave) * 1024]), koff[c]);
+  };
   auto issue_v = [&](int t, int slot) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t rv = tile_rsrc(vbase, vend, vrow_b, t);
 #pragma unroll
@@ -515,11 +540,12 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
   const float c2 = a.scale_log2;
   const DA_LDS char* lds0 = (const DA_LDS char*)&smem[0][0][0];
 
-  // S^T = K(stage) Q^T into x (raw scores): x[rg][hf] holds keys 32 hf ..
-  // 32 hf + 31 of the tile for row group rg. K fragment q (k-step q / NH of
-  // half q % NH) is read once and feeds the MFMA of every row group.
-  auto qk = [&](int stage, f32x16 (&x)[RG][NH]) __attribute__((always_inline)) {
-    const DA_LDS char* ks = lds0 + stage * (2 * TL::BYTES);
+  // S^T = K(slot) Q^T into x (raw scores), slot = 2 stage of the tile buffers:
+  // x[rg][hf] holds keys 32 hf .. 32 hf + 31 of the tile for row group rg. K
+  // fragment q (k-step q / NH of half q % NH) is read once and feeds the MFMA
+  // of every row group.
+  auto qk = [&](int slot, f32x16 (&x)[RG][NH]) __attribute__((always_inline)) {
+    const DA_LDS char* ks = lds0 + slot * TL::BYTES;
 #pragma unroll
     for (int rg = 0; rg < RG; ++rg)
 #pragma unroll
@@ -756,7 +782,7 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
 #pragma unroll
         for (int jx = 0; jx < 8 * NH; ++jx) l_i[rg] = E::add_pair(pk[rg][jx], l_i[rg]);
       }
-      if (!LAST) qk(P ^ 1, nxt);
+      if (!LAST) qk(2 * (P ^ 1), nxt);
 #pragma unroll
       for (int kk = 0; kk < 2 * NH; ++kk) {
 #pragma unroll
@@ -845,11 +871,25 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
       issue_k(0, 0);
       issue_v(0, 0);
       if (nt > 1) issue_k(1, 1);
+      // A later split of a one-round launch starts from the row max of the
+      // list's first tile, as the unsplit list would: every probability then
+      // has the same exponent offset, hence the same rounding, as in the
+      // key-sparse pass over those rows, whose rounding errors the delta
+      // composition subtracts (with a max per split the composed output of a
+      // 1531-token layer was 6 % further from 64-bit arithmetic). One more
+      // score product per item, no extra wait.
+      const bool ref = !KSPARSE && a.part_f32 && t_off > 0;
+      if (ref) issue_ref(-t_off);
       wait_vmcnt<0>();
       __syncthreads();
-      // (64 rows per wave) Q into AGPRs only now, so that the prologue waits
+      // (one wave per SIMD) Q into AGPRs only now, so that the prologue waits
       // for the Q loads and the first DMAs at once
       pin_q();
+      if (ref) {
+        qk(3, sa);
+        mask(-t_off, sa);
+        update(sa);
+      }
       qk(0, sa);
       mask(0, sa);
       update(sa);
@@ -1061,8 +1101,10 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
       store_rows16(op, o);
     }
   } else {
-    // normalised split rows O / l in the element type, a 16-byte row piece
-    // per lane after one permlane32 swap (the merge reads them back once).
+    // normalised split rows O / l for the merge, which reads them back once:
+    // as floats in the one-round launches, where a 16-bit rounding of every
+    // split would show beside that of the output, in the element type in the
+    // long ones, a 16-byte row piece per lane after one permlane32 swap.
     // At half the fp32 volume, plain stores through L2 measured 0.5-1 %
     // faster than non-temporal ones; with fp32 partials the non-temporal form
     // had kept the shared key/value chunk in L2 (split-kernel fetch 1.78 ->
@@ -1071,25 +1113,38 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
     for (int rg = 0; rg < RG; ++rg) {
       if (!valid[rg]) continue;   // the merge reads the rows of the selection only
       const int r = (RG * wave + rg) * 32 + ln;
-      uint32_t* po = a.part_o + ((int64_t)w * a.ws_rows + r) * (D / 2);
+      if (a.part_f32) {
+        float* po = (float*)a.part_o + ((int64_t)w * a.ws_rows + r) * D;
 #pragma unroll
-      for (int dt = 0; dt < NDT; ++dt)
+        for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-        for (int p2 = 0; p2 < 2; ++p2) {
-          u32x2 x0, x1;
-          const int j0 = 2 * p2, j1 = 2 * p2 + 1;
-          x0[0] = E::pack2(acc[rg][dt][4 * j0 + 0] * inv[rg], acc[rg][dt][4 * j0 + 1] * inv[rg]);
-          x0[1] = E::pack2(acc[rg][dt][4 * j0 + 2] * inv[rg], acc[rg][dt][4 * j0 + 3] * inv[rg]);
-          x1[0] = E::pack2(acc[rg][dt][4 * j1 + 0] * inv[rg], acc[rg][dt][4 * j1 + 1] * inv[rg]);
-          x1[1] = E::pack2(acc[rg][dt][4 * j1 + 2] * inv[rg], acc[rg][dt][4 * j1 + 3] * inv[rg]);
+          for (int jq = 0; jq < 4; ++jq) {
+            f32x4 x;
 #pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            auto sw = __builtin_amdgcn_permlane32_swap(x0[e], x1[e], false, false);
-            x0[e] = sw[0];
-            x1[e] = sw[1];
+            for (int e = 0; e < 4; ++e) x[e] = acc[rg][dt][4 * jq + e] * inv[rg];
+            *(f32x4*)(po + 32 * dt + 8 * jq + 4 * lg) = x;
           }
-          *(u32x4*)(po + (32 * dt + 16 * p2 + 8 * lg) / 2) = (u32x4){x0[0], x0[1], x1[0], x1[1]};
-        }
+      } else {
+        uint32_t* po = (uint32_t*)a.part_o + ((int64_t)w * a.ws_rows + r) * (D / 2);
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+          for (int p2 = 0; p2 < 2; ++p2) {
+            u32x2 x0, x1;
+            const int j0 = 2 * p2, j1 = 2 * p2 + 1;
+            x0[0] = E::pack2(acc[rg][dt][4 * j0 + 0] * inv[rg], acc[rg][dt][4 * j0 + 1] * inv[rg]);
+            x0[1] = E::pack2(acc[rg][dt][4 * j0 + 2] * inv[rg], acc[rg][dt][4 * j0 + 3] * inv[rg]);
+            x1[0] = E::pack2(acc[rg][dt][4 * j1 + 0] * inv[rg], acc[rg][dt][4 * j1 + 1] * inv[rg]);
+            x1[1] = E::pack2(acc[rg][dt][4 * j1 + 2] * inv[rg], acc[rg][dt][4 * j1 + 3] * inv[rg]);
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+              auto sw = __builtin_amdgcn_permlane32_swap(x0[e], x1[e], false, false);
+              x0[e] = sw[0];
+              x1[e] = sw[1];
+            }
+            *(u32x4*)(po + (32 * dt + 16 * p2 + 8 * lg) / 2) = (u32x4){x0[0], x0[1], x1[0], x1[1]};
+          }
+      }
       if (lg == 0) {
         a.part_ml[(int64_t)w * 2 * a.ws_rows + r] = m_i[rg];
         a.part_ml[(int64_t)w * 2 * a.ws_rows + a.ws_rows + r] = l_tot[rg];
@@ -1115,7 +1170,8 @@ struct MergeArgs {
   int window, sink;
   int lanes;        // P: threads sharing one (row, 8-column) task, splits s = p mod P
   int wgs;          // workgroups per row tile
-  const uint32_t* part_o;   // element pairs of O / l per split row
+  int vis, slots;           // as in AttnArgs
+  const void* part_o;       // O / l per split row (as in AttnArgs)
   const float* part_ml;
   int ws_rows;      // as in AttnArgs
   int bm;           // as in AttnArgs: flattened rows per row tile of the split launch
@@ -1132,18 +1188,21 @@ struct MergeArgs {
   float* lse;
 };
 
-template <typename T, int D>
+// F32: the partials are floats (AttnArgs::part_f32).
+template <typename T, int D, bool F32>
 __global__ __launch_bounds__(MTHR) void qsparse_merge_kernel(MergeArgs a) {
   using E = Elt<T>;
   constexpr int CPR = D / 8;   // 8-column chunks per row
   __shared__ int s_hmax[4], s_lmin[4];
   int tile = blockIdx.x / a.wgs;
   const int sub = blockIdx.x % a.wgs;
+  int chunk = a.chunk;
   if (a.n_rows_dev) {
     // live row tiles of every (b, kv head) first, as the split items
     const int n_live = min(max(*a.n_rows_dev, 0), a.n_rows);
     const int mt_live = (n_live * a.G + a.bm - 1) / a.bm;
     if (mt_live == 0 || tile >= a.B * a.Hkv * mt_live) return;
+    chunk = live_chunk(chunk, a.B * a.Hkv * mt_live, a.vis, a.slots);
     tile = (tile / mt_live) * a.n_mtiles + tile % mt_live;
   }
   const int mt = tile % a.n_mtiles;
@@ -1180,7 +1239,7 @@ __global__ __launch_bounds__(MTHR) void qsparse_merge_kernel(MergeArgs a) {
   int n_first, second_t0, n_second;
   tile_list(hi_max, lo_min, a.window > 0 ? a.sink : 0, n_first, second_t0, n_second);
   const int n_list = n_first + n_second;
-  const int chunk = a.n_kv_dev ? max(1, (n_list + a.n_splits - 1) / a.n_splits) : a.chunk;
+  if (a.n_kv_dev) chunk = max(1, (n_list + a.n_splits - 1) / a.n_splits);
   const int nsv = (n_list + chunk - 1) / chunk;
 
   const size_t esz = sizeof(T);
@@ -1215,8 +1274,9 @@ __global__ __launch_bounds__(MTHR) void qsparse_merge_kernel(MergeArgs a) {
       M = mn;
     };
     for (int s0 = p; s0 < nsv; s0 += MU * P) {
+      constexpr int NX = F32 ? 2 : 1;
       float ms[MU], ls[MU];
-      u32x4 xs[MU];
+      u32x4 xs[MU][NX];
 #pragma unroll
       for (int u = 0; u < MU; ++u) {
         const int s = s0 + u * P;
@@ -1224,11 +1284,14 @@ __global__ __launch_bounds__(MTHR) void qsparse_merge_kernel(MergeArgs a) {
           const int64_t w = ((int64_t)bh * a.n_splits + s) * a.n_mtiles + mt;
           ms[u] = a.part_ml[w * 2 * a.ws_rows + r];
           ls[u] = a.part_ml[w * 2 * a.ws_rows + a.ws_rows + r];
-          xs[u] = *(const u32x4*)(a.part_o + (w * a.ws_rows + r) * (D / 2) + 4 * c);
+          const u32x4* px = (const u32x4*)((const char*)a.part_o + (w * a.ws_rows + r) * (D * (F32 ? 4 : 2))) + NX * c;
+#pragma unroll
+          for (int x = 0; x < NX; ++x) xs[u][x] = px[x];
         } else {
           ms[u] = NEG_BIG;
           ls[u] = 0.f;
-          xs[u] = (u32x4){0, 0, 0, 0};
+#pragma unroll
+          for (int x = 0; x < NX; ++x) xs[u][x] = (u32x4){0, 0, 0, 0};
         }
       }
 #pragma unroll
@@ -1236,8 +1299,13 @@ __global__ __launch_bounds__(MTHR) void qsparse_merge_kernel(MergeArgs a) {
         float o[8];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          o[2 * e] = E::lo(xs[u][e]);
-          o[2 * e + 1] = E::hi(xs[u][e]);
+          if constexpr (F32) {
+            o[e] = __uint_as_float(xs[u][0][e]);
+            o[4 + e] = __uint_as_float(xs[u][1][e]);
+          } else {
+            o[2 * e] = E::lo(xs[u][0][e]);
+            o[2 * e + 1] = E::hi(xs[u][0][e]);
+          }
         }
         take(ms[u], ls[u], o);
       }
@@ -1308,6 +1376,8 @@ struct QsparsePlan {
   int ws_rows;      // workspace rows per item: a tile's valid (row, head) pairs at most
   int bm;           // flattened (row, head) pairs per row tile of the split launch
   size_t ws_bytes;
+  int64_t vis;      // bound of a row tile's list
+  bool f32;         // float partials
 };
 
 // Rows per workgroup of a launch: for the head_dim-128 key-sparse launches
@@ -1325,17 +1395,24 @@ static int rows_bm(int D) { return D == 128 ? bm_of(DA_RG_ROWS) : bm_of(1); }
 // lanes per task, 256 threads each.
 constexpr int64_t MERGE_WGS_MAX = (int64_t)BM_MAX * (256 / 8) * 16 / MTHR;
 
+// Workspace bytes per split row: O / l, max and sum.
+static size_t part_row_bytes(const QsparsePlan& p, int D) {
+  return D * (p.f32 ? sizeof(float) : sizeof(uint16_t)) + 2 * sizeof(float);
+}
+
 // Split plan over the tile lists: `vis` bounds a row tile's list length, each
 // item takes `chunk` consecutive tiles of it (at least `min_chunk`); `target`
 // items in total.
 static QsparsePlan plan_qsparse(int B, int Hq, int Hkv, int n, int64_t vis, int D, int target,
-                                int min_chunk, int bm, int max_chunk = 0x7fffffff) {
+                                int min_chunk, int bm, int max_chunk = 0x7fffffff, bool f32 = false) {
   QsparsePlan p;
+  p.f32 = f32;
   const int G = Hq / Hkv;
   p.bm = bm;
   p.n_mtiles = (int)(((int64_t)n * G + bm - 1) / bm);
   const int64_t base = (int64_t)B * Hkv * p.n_mtiles;
   if (vis < 1) vis = 1;
+  p.vis = vis;
   int64_t want = (target + base - 1) / base;
   if (want < 1) want = 1;
   if (want > vis) want = vis;
@@ -1349,33 +1426,72 @@ static QsparsePlan plan_qsparse(int B, int Hq, int Hkv, int n, int64_t vis, int 
   const bool fits = items <= 0x7fffff00LL && base * MERGE_WGS_MAX <= 0x7fffff00LL;
   p.n_items = fits ? (int)items : 0;
   p.ws_rows = (int)min((int64_t)bm, (int64_t)n * G);
-  p.ws_bytes = fits ? (size_t)p.n_items * p.ws_rows * (D * sizeof(uint16_t) + 2 * sizeof(float)) : 0;
+  p.ws_bytes = fits ? (size_t)p.n_items * p.ws_rows * part_row_bytes(p, D) : 0;
   return p;
 }
 
-// Causal selected rows: ~8192 items (about half of them past the end of a
-// causal row tile's list), but at least 56 key tiles each: short items pay
-// their prologue and partials, and at 32K keys (638 rows x 32 heads) 56 packs
-// the ~1K useful items into two rounds of resident workgroups (0.258 ms vs
-// 0.269-0.272 at 40; neutral at 128K keys, where the 8K target binds).
-// A short row list (fewer than 64 (batch, kv head, row tile) triples: the
-// adaptive stride's chunks, a dense tail alone) cannot fill the GPU with
-// 56-tile items, and one item's latency would bound the launch: ~1024 items of
-// at least 16 tiles instead.
-static QsparsePlan plan_rows(int B, int Hq, int Hkv, int n, int Skv, int D) {
+// Workgroups of a launch that run at once on the 256 CUs.
+static int64_t resident_slots(int D) { return 256 * attn_occupancy(D, 1); }
+
+// Split plan of a selected-rows launch.
+//
+// One round: when the row tiles' whole lists, cut into as many splits as the
+// resident slots hold, give items of at most 80 key tiles, that cut is the
+// plan: every slot takes one item and no second round runs half empty
+// (measured against the 56-tile items below: 268 rows of 32 heads at 6001 keys
+// 76 -> 46 us, 128 rows at 65000 keys 177 -> 143 us, 509 rows at head_dim 256
+// and 16901 keys 217 -> 141 us). Above 80 tiles the lists of anchor rows,
+// half of them short, leave too many slots idle (638 rows at 32768 keys: 263
+// us in one round of 171-tile items, 236 us at 56 tiles); rows that end a
+// sequence (a prompt chunk, no q_rows) see nearly all keys and take up to 160
+// tiles if the round is at least 95 % full (2000 rows at head_dim 64 and
+// 40000 keys 208 -> 183 us). Their items hold at least sqrt(0.35 list) tiles:
+// a split costs the merge about a third of a key tile's time (40 rows of 32
+// heads at 8000 keys: 24.7 / 25.5 / 22.7 / 23.8 us at 4 / 5 / 8 / 10 tiles).
+// Selected rows (q_rows) take at least 4 whatever the list, so that a row's
+// splits, and with them its bits, are the same in a launch over a prefix of
+// the keys (226 rows of 8 heads at 1531 keys 23.3 -> 14.5 us).
+//
+// Longer launches: ~8192 items (about half of them past the end of a causal
+// row tile's list), but at least 56 key tiles each: short items pay their
+// prologue and partials, and at 32K keys (638 rows x 32 heads) 56 packs the
+// ~1K useful items into two rounds of resident workgroups (0.258 ms vs
+// 0.269-0.272 at 40; neutral at 128K keys, where the 8K target binds). A
+// short row list (fewer than 64 (batch, kv head, row tile) triples) takes
+// ~1024 items of at least 16 tiles instead, since 56-tile items cannot fill
+// the GPU.
+static QsparsePlan plan_rows(int B, int Hq, int Hkv, int n, int Skv, int D, bool ends_seq) {
   const int64_t vis = (Skv + BN - 1) / BN;
   const int bm = rows_bm(D);
   const int64_t tiles = (int64_t)B * Hkv * (((int64_t)n * (Hq / Hkv) + bm - 1) / bm);
+  const int64_t slots = resident_slots(D), per_tile = tiles > 0 ? slots / tiles : 0;
+  if (per_tile > 0) {
+    const int64_t chunk = (vis + per_tile - 1) / per_tile;
+    if (chunk <= 80 || (ends_seq && chunk <= 160 && 20 * tiles * per_tile >= 19 * slots)) {
+      int least = ends_seq ? 1 : 4;
+      while (ends_seq && 20 * (int64_t)least * least < 7 * vis) ++least;
+      return plan_qsparse(B, Hq, Hkv, n, vis, D, (int)(tiles * per_tile), least, bm, 0x7fffffff, true);
+    }
+  }
   if (tiles < 64) return plan_qsparse(B, Hq, Hkv, n, vis, D, 1024, 16, bm);
   return plan_qsparse(B, Hq, Hkv, n, vis, D, DA_ROWS_ITEMS, DA_ROWS_MIN_TILES, bm, DA_ROWS_MAX_TILES);
+}
+
+// Workspace of a selected-rows launch: the larger of its two plans (the
+// query does not tell whether the rows end the sequence).
+static size_t rows_ws_bytes(int B, int Hq, int Hkv, int n, int Skv, int D) {
+  const QsparsePlan p = plan_rows(B, Hq, Hkv, n, Skv, D, false);
+  const QsparsePlan e = plan_rows(B, Hq, Hkv, n, Skv, D, true);
+  return p.n_items <= 0 || e.n_items <= 0 ? 0 : p.ws_bytes > e.ws_bytes ? p.ws_bytes : e.ws_bytes;
 }
 
 // Split plan for n rows of which about n_live hold keys (the others are -1
 // rows with empty tile lists: the adaptive stride's padded row lists): the
 // items per row tile follow the plan of n_live rows, the grid covers all n.
-static QsparsePlan plan_rows_live(int B, int Hq, int Hkv, int n, int n_live, int Skv, int D) {
-  if (n_live >= n || n_live < 1) return plan_rows(B, Hq, Hkv, n, Skv, D);
-  QsparsePlan p = plan_rows(B, Hq, Hkv, n_live, Skv, D);
+static QsparsePlan plan_rows_live(int B, int Hq, int Hkv, int n, int n_live, int Skv, int D,
+                                  bool ends_seq) {
+  if (n_live >= n || n_live < 1) return plan_rows(B, Hq, Hkv, n, Skv, D, ends_seq);
+  QsparsePlan p = plan_rows(B, Hq, Hkv, n_live, Skv, D, false);
   const int G = Hq / Hkv;
   p.n_mtiles = (int)(((int64_t)n * G + p.bm - 1) / p.bm);
   const int64_t base = (int64_t)B * Hkv * p.n_mtiles;
@@ -1383,7 +1499,7 @@ static QsparsePlan plan_rows_live(int B, int Hq, int Hkv, int n, int n_live, int
   const bool fits = p.n_items > 0 && items <= 0x7fffff00LL && base * MERGE_WGS_MAX <= 0x7fffff00LL;
   p.n_items = fits ? (int)items : 0;
   p.ws_rows = (int)min((int64_t)p.bm, (int64_t)n * G);
-  p.ws_bytes = fits ? (size_t)p.n_items * p.ws_rows * (D * sizeof(uint16_t) + 2 * sizeof(float)) : 0;
+  p.ws_bytes = fits ? (size_t)p.n_items * p.ws_rows * part_row_bytes(p, D) : 0;
   return p;
 }
 
@@ -1425,8 +1541,9 @@ static void dispatch_attn(const AttnArgs& a, int D, int dtype, hipStream_t s) {
 }
 
 template <typename T, int D>
-static void launch_merge(const MergeArgs& m, int n_tiles, hipStream_t s) {
-  hipLaunchKernelGGL((qsparse_merge_kernel<T, D>), dim3(n_tiles), dim3(MTHR), 0, s, m);
+static void launch_merge(const MergeArgs& m, int n_tiles, bool f32, hipStream_t s) {
+  if (f32) hipLaunchKernelGGL((qsparse_merge_kernel<T, D, true>), dim3(n_tiles), dim3(MTHR), 0, s, m);
+  else hipLaunchKernelGGL((qsparse_merge_kernel<T, D, false>), dim3(n_tiles), dim3(MTHR), 0, s, m);
 }
 
 // Query heads per key-sparse row tile: bm / 64 heads (64-row tiles) when
@@ -1637,8 +1754,10 @@ static int run_qsparse(const QsparsePlan& p, const void* q, const void* k, const
   a.chunk = p.chunk; a.n_splits = p.n_splits; a.n_kv_dev = n_kv_dev;
   a.n_rows_dev = n_rows_dev;
   a.window = window; a.sink = sink;
-  a.part_o = (uint32_t*)workspace;
-  a.part_ml = (float*)((char*)workspace + (size_t)p.n_items * p.ws_rows * D * sizeof(uint16_t));
+  a.vis = (int)p.vis; a.slots = (int)resident_slots(D);
+  a.part_o = workspace; a.part_f32 = p.f32;
+  a.part_ml = (float*)((char*)workspace +
+                       (size_t)p.n_items * p.ws_rows * D * (p.f32 ? sizeof(float) : sizeof(uint16_t)));
   a.ws_rows = p.ws_rows;
 
   MergeArgs m = {};
@@ -1647,7 +1766,9 @@ static int run_qsparse(const QsparsePlan& p, const void* q, const void* k, const
   m.n_splits = p.n_splits; m.chunk = p.chunk; m.n_kv_dev = n_kv_dev;
   m.B = B; m.n_rows_dev = n_rows_dev;
   m.window = window; m.sink = sink;
-  // P threads per (row, column chunk) task: about 4 splits each, up to 16,
+  // P threads per (row, column chunk) task: about 4 splits each, 4 to 16
+  // (at least 4 however few splits the plan has: a row's order of summation
+  // then depends on its own list, not on the keys the launch was planned for),
   // but no more threads than about half the GPU holds (2^18): a merge with
   // that many tasks already has enough loads in flight with one lane each,
   // and more lanes only add rounds of waves (128K layer: 36 us at one lane
@@ -1656,11 +1777,12 @@ static int run_qsparse(const QsparsePlan& p, const void* q, const void* k, const
   {
     const int64_t rows = min((int64_t)p.bm, (int64_t)n * a.G);
     const int64_t tasks = (int64_t)B * Hkv * p.n_mtiles * rows * (D / 8);
-    m.lanes = 1;
+    m.lanes = 4;
     while (m.lanes < 16 && m.lanes * 4 < p.n_splits) m.lanes <<= 1;
     while (m.lanes > 1 && tasks * m.lanes > (1 << 18)) m.lanes >>= 1;
     m.wgs = (int)((rows * (D / 8) * m.lanes + MTHR - 1) / MTHR);
   }
+  m.vis = a.vis; m.slots = a.slots;
   m.part_o = a.part_o; m.part_ml = a.part_ml; m.ws_rows = p.ws_rows; m.bm = p.bm;
   m.epi = epi; m.n_anchor = (epi == DA_EPI_DELTA || epi == DA_EPI_DENSE) ? n_anchor : 0;
   m.o = o; m.os_b = o_str[0]; m.os_h = o_str[1]; m.os_s = o_str[2];
@@ -1675,15 +1797,15 @@ static int run_qsparse(const QsparsePlan& p, const void* q, const void* k, const
   dispatch_attn<MODE_QSPARSE>(a, D, dtype, s);
   const int n_tiles = B * Hkv * p.n_mtiles * m.wgs;
   if (dtype == DA_BF16) {
-    if (D == 128) launch_merge<__bf16, 128>(m, n_tiles, s);
-    else if (D == 64) launch_merge<__bf16, 64>(m, n_tiles, s);
-    else if (D == 256) launch_merge<__bf16, 256>(m, n_tiles, s);
-    else launch_merge<__bf16, 32>(m, n_tiles, s);
+    if (D == 128) launch_merge<__bf16, 128>(m, n_tiles, p.f32, s);
+    else if (D == 64) launch_merge<__bf16, 64>(m, n_tiles, p.f32, s);
+    else if (D == 256) launch_merge<__bf16, 256>(m, n_tiles, p.f32, s);
+    else launch_merge<__bf16, 32>(m, n_tiles, p.f32, s);
   } else {
-    if (D == 128) launch_merge<_Float16, 128>(m, n_tiles, s);
-    else if (D == 64) launch_merge<_Float16, 64>(m, n_tiles, s);
-    else if (D == 256) launch_merge<_Float16, 256>(m, n_tiles, s);
-    else launch_merge<_Float16, 32>(m, n_tiles, s);
+    if (D == 128) launch_merge<_Float16, 128>(m, n_tiles, p.f32, s);
+    else if (D == 64) launch_merge<_Float16, 64>(m, n_tiles, p.f32, s);
+    else if (D == 256) launch_merge<_Float16, 256>(m, n_tiles, p.f32, s);
+    else launch_merge<_Float16, 32>(m, n_tiles, p.f32, s);
   }
   return hipGetLastError() == hipSuccess ? DA_OK : DA_ERR_LAUNCH;
 }
@@ -1692,7 +1814,7 @@ extern "C" size_t da_qsparse_workspace_bytes(int B, int Hq, int Hkv, int n, int 
   if (B < 1 || Hq < 1 || Hkv < 1 || Hq % Hkv != 0 || n < 1 || Skv < 1 ||
       !head_dim_ok(D))
     return 0;
-  return plan_rows(B, Hq, Hkv, n, Skv, D).ws_bytes;
+  return rows_ws_bytes(B, Hq, Hkv, n, Skv, D);
 }
 
 static int qsparse_fwd(const void* q, const void* k, const void* v,
@@ -1722,7 +1844,7 @@ static int qsparse_fwd(const void* q, const void* k, const void* v,
       !strides8(q_str) || !strides8(k_str) || !strides8(v_str) || !strides8(o_str))
     return DA_ERR_ALIGNMENT;
   if (!kv_rows_ok(k_str, v_str)) return DA_ERR_INVALID_ARG;
-  const QsparsePlan p = plan_rows_live(B, Hq, Hkv, n, n_live, Skv, D);
+  const QsparsePlan p = plan_rows_live(B, Hq, Hkv, n, n_live, Skv, D, q_rows == nullptr);
   return run_qsparse(p, q, k, v, q_rows, row_last, rl_bstride, n, B, Hq, Hkv, Sq, Skv, D,
                      q_str, k_str, v_str, o, o_str, epi, n_anchor, delta, d_str, 0, 0,
                      sm_scale, workspace, workspace_bytes, dtype, stream, nullptr, nullptr,
@@ -1747,7 +1869,8 @@ extern "C" size_t da_qsparse_workspace_bytes_live(int B, int Hq, int Hkv, int n,
   if (B < 1 || Hq < 1 || Hkv < 1 || Hq % Hkv != 0 || n < 1 || n_live < 1 || Skv < 1 ||
       !head_dim_ok(D))
     return 0;
-  return plan_rows_live(B, Hq, Hkv, n, n_live, Skv, D).ws_bytes;
+  if (n_live >= n) return rows_ws_bytes(B, Hq, Hkv, n, Skv, D);
+  return plan_rows_live(B, Hq, Hkv, n, n_live, Skv, D, false).ws_bytes;
 }
 
 extern "C" int da_qsparse_attn_fwd_live(const void* q, const void* k, const void* v,

@@ -1,0 +1,41 @@
+"""Selected-rows launches at the edges of their split plan: lists of one tile,
+lists cut into the shortest items, a plan of exactly one item per resident
+workgroup, one item per row tile, and the longest items of rows that end the
+sequence; against the oracle (tolerance: the layer's parity bar)."""
+
+import pytest
+import torch
+
+from helpers import assert_close, gen_qkv, np64
+from oracle import delta_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,H,Hkv,n,N,D", [
+    (1, 2, 2, 5, 40, 64),         # one key tile
+    (1, 8, 2, 17, 600, 64),       # the shortest items: two of ten tiles
+    (1, 8, 2, 33, 8000, 128),     # seven-tile items of 125
+    (1, 8, 8, 1000, 1100, 128),   # 64 row tiles, eight splits: every slot one item
+    (1, 8, 8, 1000, 1100, 256),   # the same at one workgroup per CU: four splits
+    (64, 8, 8, 2, 1200, 32),      # 512 row tiles: one item each
+    (65, 8, 8, 2, 1200, 32),      # one row tile past the slots
+    (64, 8, 8, 2, 5200, 32),      # rows that end the sequence, one 82-tile item each
+])
+@pytest.mark.parametrize("selected", [False, True])
+def test_plan_edges(gpu, B, H, Hkv, n, N, D, selected):
+    """The same rows as the last n rows of a sequence (no q_rows) and as rows
+    selected from a full q; both plans against the oracle on two batches."""
+    from delta_attention import ops
+    q, k, v = gen_qkv(B, H, Hkv, n, D, seed=N + D, N=N)
+    rows = torch.arange(N - n, N, device="cuda")
+    if selected:
+        full = torch.zeros(B, H, N, D, dtype=q.dtype, device="cuda")
+        full[:, :, N - n:] = q
+        out = ops.qsparse_attention(full, k, v, rows, D ** -0.5, q_rows=rows)
+    else:
+        out = ops.qsparse_attention(q, k, v, rows[None], D ** -0.5)
+    for b in {0, B - 1}:
+        ref = O.qsparse_attention(np64(q[b:b + 1]), np64(k[b:b + 1]), np64(v[b:b + 1]),
+                                  rows.cpu().numpy(), D ** -0.5)
+        assert_close(np64(out[b:b + 1]), ref, what=f"B{B} n{n} N{N} D{D} batch {b}")
