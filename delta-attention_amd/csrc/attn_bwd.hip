@@ -49,8 +49,9 @@ constexpr int BM = 32 * NWAVE;   // dq kernel: flattened (row, head) pairs per w
 // dq kernel: keys per tile (at head_dim 128 computed as two 32-key halves one
 // after the other, which keeps the score registers small enough for two waves
 // per SIMD)
+constexpr int DQ_BN = 64;
 template <int D>
-constexpr int dq_bn() { return 64; }
+constexpr int dq_bn() { return DQ_BN; }
 constexpr int KT = 32 * NWAVE;   // dkdv kernel: keys per workgroup
 constexpr int RT = 32;           // dkdv kernel: rows per step
 constexpr int RPC_MAX = 8192;    // dkdv kernel: rows per chunk at most (default)
@@ -284,6 +285,7 @@ __global__ __launch_bounds__(NTHR, 2) void dq_kernel(BwdArgs a) {
   int nt = n_first + n_second;
   const int t_off = split * a.chunk;
   nt = max(0, min(a.chunk, nt - t_off));
+  if (nt == 0 && a.n_splits > 1) return;   // past the list: the reduce skips this split
 
   const char* kbase = (const char*)a.k + ((int64_t)b * a.ks_b + (int64_t)hk * a.ks_h) * esz;
   const char* vbase = (const char*)a.v + ((int64_t)b * a.vs_b + (int64_t)hk * a.vs_h) * esz;
@@ -450,7 +452,14 @@ __global__ __launch_bounds__(RED) void dq_reduce_kernel(BwdArgs a) {
   float s[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) s[e] = 0.f;
-  for (int sp = 0; sp < a.n_splits; ++sp) {
+  // the splits of this row tile's list, whose last row sees the most keys
+  int nsv = a.n_splits;
+  if (ROWS) {
+    const int64_t lim = min(a.row_last[min((mt * BM + BM - 1) / a.G, a.n_rows - 1)], (int64_t)(a.n_kv - 1));
+    const int list = lim < 0 ? 0 : (int)lim / dq_bn<D>() + 1;
+    nsv = min(nsv, (list + a.chunk - 1) / a.chunk);
+  }
+  for (int sp = 0; sp < nsv; ++sp) {
     const int64_t w = ((int64_t)bh * a.n_splits + sp) * a.n_mtiles + mt;
     const f32x4* p = (const f32x4*)(a.dq_part + (w * BM + r) * D + 8 * c);
     const f32x4 x0 = p[0], x1 = p[1];
@@ -1018,7 +1027,12 @@ struct DqPlan {
 };
 
 // Key tiles per dq item: key-sparse rows take their whole (window-sized)
-// list; selected rows split lists longer than 64 tiles into about 4096 items.
+// list; selected rows split theirs so that the items fill one round of the 512
+// resident workgroups, 4 to 64 tiles each (190 rows of 32 heads at 4096 keys:
+// backward of the rows 180 -> 86 us; 248 rows of 8 heads at 2048 keys 84 -> 55
+// us), or, where that round would need longer items, into about 4096 items of
+// at least 64 tiles (638 rows at 32768 keys: 950 us at 64 and at 128 tiles,
+// 1002 at 20). Items past the end of a short list write nothing.
 DqPlan plan_dq(int B, int Hkv, int G, int n_rows, int64_t list_tiles, bool rows) {
   DqPlan p;
   p.n_mtiles = (int)(((int64_t)n_rows * G + BM - 1) / BM);
@@ -1028,13 +1042,14 @@ DqPlan plan_dq(int B, int Hkv, int G, int n_rows, int64_t list_tiles, bool rows)
     return p;
   }
   if (list_tiles < 1) list_tiles = 1;
-  int64_t want = 1;
-  if (list_tiles > 64) {
-    const int64_t base = (int64_t)B * Hkv * p.n_mtiles;
-    want = (4096 + base - 1) / base;
-    want = std::min<int64_t>(std::max<int64_t>(want, 1), (list_tiles + 63) / 64);
+  const int64_t base = (int64_t)B * Hkv * p.n_mtiles;
+  const int64_t one = std::max<int64_t>(512 / base, 1);          // splits of one round
+  int64_t chunk = std::max<int64_t>((list_tiles + one - 1) / one, 4);
+  if (chunk > 64) {
+    const int64_t want = (4096 + base - 1) / base;
+    chunk = std::max<int64_t>((list_tiles + want - 1) / want, 64);
   }
-  p.chunk = (int)((list_tiles + want - 1) / want);
+  p.chunk = (int)std::min(chunk, list_tiles);
   p.n_splits = (int)((list_tiles + p.chunk - 1) / p.chunk);
   return p;
 }
@@ -1052,10 +1067,9 @@ static std::atomic<int> g_rpc_max{RPC_MAX};
 // (window 4096: 4096 + 128 rows), each a whole item with its K/V loads and
 // dK/dV partials (Qwen3 64K x 2 backward 102 ms; 66 ms with one 4224-row
 // chunk per block).
-KvPlan plan_kv(int n_rows, int n_kv, int window, int sink, bool rows) {
+KvPlan plan_kv_cap(int n_rows, int n_kv, int window, int sink, bool rows, int64_t cap) {
   KvPlan p;
   p.n_blk = (n_kv + KT - 1) / KT;
-  const int64_t cap = g_rpc_max.load(std::memory_order_relaxed);
   auto up = [](int64_t x) { return (int)(((x + RT - 1) / RT) * RT); };
   auto split = [&](int64_t span, int& rpc, int& n) {
     span = std::max<int64_t>(span, 1);
@@ -1075,6 +1089,22 @@ KvPlan plan_kv(int n_rows, int n_kv, int window, int sink, bool rows) {
   }
   p.items_per_bh = p.nsb * p.ncs + (p.n_blk - p.nsb) * p.nco;
   p.part_per_bh = p.nco > 1 ? p.items_per_bh : p.ncs > 1 ? p.nsb * p.ncs : 0;
+  return p;
+}
+
+// Few key blocks (short sequences, few heads) leave CUs idle with one item a
+// block: the smallest chunks, of at least 96 rows, whose items still fit the
+// 256 workgroups that run at once (one per CU). Key-sparse backward of 8 / 2
+// heads x 2 batches at 2048 rows 98 -> 65 us, of 32 / 4 heads at 1024 rows 220
+// -> 84 us; their selected rows 84 -> 75 and 100 -> 85 us.
+KvPlan plan_kv(int bh, int n_rows, int n_kv, int window, int sink, bool rows) {
+  const int64_t cap = g_rpc_max.load(std::memory_order_relaxed);
+  KvPlan p = plan_kv_cap(n_rows, n_kv, window, sink, rows, cap);
+  if ((int64_t)bh * p.items_per_bh >= 256) return p;
+  for (int64_t rpc = 96; rpc < p.rpc; rpc += RT) {
+    const KvPlan c = plan_kv_cap(n_rows, n_kv, window, sink, rows, rpc);
+    if ((int64_t)bh * c.items_per_bh <= 256) return c;
+  }
   return p;
 }
 
@@ -1186,7 +1216,7 @@ extern "C" size_t da_sparse_attn_bwd_workspace_bytes(int B, int Hq, int Hkv, int
       sink < 0 || (D != 32 && D != 64 && D != 128))
     return 0;
   const DqPlan dq = plan_dq(B, Hkv, Hq / Hkv, S, 0, false);
-  const KvPlan kv = plan_kv(S, S, window, sink, false);
+  const KvPlan kv = plan_kv(B * Hkv, S, S, window, sink, false);
   return bwd_ws_bytes(B, Hq, Hkv, S, S, D, dq, kv, false);
 }
 
@@ -1194,9 +1224,8 @@ extern "C" size_t da_qsparse_attn_bwd_workspace_bytes(int B, int Hq, int Hkv, in
   if (B < 1 || Hq < 1 || Hkv < 1 || Hq % Hkv != 0 || n < 1 || Skv < 1 ||
       (D != 32 && D != 64 && D != 128))
     return 0;
-  const int bn = D == 128 ? 32 : 64;
-  const DqPlan dq = plan_dq(B, Hkv, Hq / Hkv, n, ((int64_t)Skv + bn - 1) / bn, true);
-  const KvPlan kv = plan_kv(n, Skv, 0, 0, true);
+  const DqPlan dq = plan_dq(B, Hkv, Hq / Hkv, n, ((int64_t)Skv + DQ_BN - 1) / DQ_BN, true);
+  const KvPlan kv = plan_kv(B * Hkv, n, Skv, 0, 0, true);
   return bwd_ws_bytes(B, Hq, Hkv, n, Skv, D, dq, kv, true);
 }
 
@@ -1236,7 +1265,7 @@ extern "C" int da_sparse_attn_bwd(const void* q, const void* k, const void* v, c
   if (rc != DA_OK) return rc;
   a.window = window; a.sink = sink; a.q_block = q_block;
   const DqPlan dqp = plan_dq(B, Hkv, a.G, S, 0, false);
-  const KvPlan kvp = plan_kv(S, S, window, sink, false);
+  const KvPlan kvp = plan_kv(B * Hkv, S, S, window, sink, false);
   const size_t need = bwd_ws_bytes(B, Hq, Hkv, S, S, D, dqp, kvp, false);
   if (!workspace || workspace_bytes < need) return DA_ERR_WORKSPACE;
   if (!aligned16(workspace)) return DA_ERR_ALIGNMENT;
@@ -1269,9 +1298,8 @@ extern "C" int da_qsparse_attn_bwd(const void* q, const void* k, const void* v, 
   // with 32-bit byte offsets (else it stages them through registers)
   a.q32 = (uint64_t)a.n_q * (uint64_t)a.qs_s * 2u <= 0xfffff000ull;
   a.window = 0; a.sink = 0; a.q_block = 1;
-  const int bn = D == 128 ? 32 : 64;
-  const DqPlan dqp = plan_dq(B, Hkv, a.G, n, ((int64_t)Skv + bn - 1) / bn, true);
-  const KvPlan kvp = plan_kv(n, Skv, 0, 0, true);
+  const DqPlan dqp = plan_dq(B, Hkv, a.G, n, ((int64_t)Skv + DQ_BN - 1) / DQ_BN, true);
+  const KvPlan kvp = plan_kv(B * Hkv, n, Skv, 0, 0, true);
   const size_t need = bwd_ws_bytes(B, Hq, Hkv, n, Skv, D, dqp, kvp, true);
   if (!workspace || workspace_bytes < need) return DA_ERR_WORKSPACE;
   if (!aligned16(workspace)) return DA_ERR_ALIGNMENT;
