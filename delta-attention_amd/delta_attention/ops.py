@@ -8,6 +8,7 @@ synchronises.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import functools
 from typing import Optional, Tuple
@@ -29,17 +30,35 @@ def _code(t: torch.Tensor) -> int:
 def _ready(t: torch.Tensor) -> torch.Tensor:
     """Rows contiguous and 16-byte aligned, as the kernels read them; other
     dimensions keep their strides (no copy for the usual transposed views)."""
-    ok = (t.stride(-1) == 1 and t.data_ptr() % 16 == 0
-          and all(s % 8 == 0 for s in t.stride()[:-1]))
-    return t if ok else t.contiguous()
+    st = t.stride()
+    bits = 0
+    for x in st[:-1]:
+        bits |= x
+    return t if st[-1] == 1 and not bits & 7 and t.data_ptr() % 16 == 0 else t.contiguous()
 
 
-def _ptr(t: Optional[torch.Tensor]):
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+# A small launch is shorter than the Python around it (one decode row: 15 us
+# of GPU time, 26 us of host time), so the helpers below keep to one cheap
+# call each: plain integers for pointers and streams (the bindings' argtypes
+# convert them), one stride() per tensor, and no device switch when the
+# tensors' device is already current.
+
+def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
+    return None if t is None else t.data_ptr()
 
 
-def _stream(dev: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+def _stream(dev: torch.device) -> int:
+    """torch's current stream of `dev` (the raw hipStream_t)."""
+    return torch._C._cuda_getCurrentRawStream(dev.index)
+
+
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def _device(dev: torch.device):
+    """`dev` as the current device: torch.cuda.device(dev), or nothing where
+    it is current already."""
+    return _SAME_DEVICE if torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
 
 
 def _on_gpu(*ts: torch.Tensor) -> torch.device:
@@ -48,6 +67,11 @@ def _on_gpu(*ts: torch.Tensor) -> torch.device:
         assert t.is_cuda, "delta-attention kernels need GPU tensors"
         assert t.device == dev, "all tensors must be on one device"
     return dev
+
+
+def _s3(t: torch.Tensor, a: int, b: int, c: int):
+    st = t.stride()
+    return L.I64x3(st[a], st[b], st[c])
 
 
 # ---------------------------------------------------------------------------
@@ -78,11 +102,11 @@ def sparse_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, windo
         out = torch.empty((B, S, H, D), device=dev, dtype=q.dtype)
     assert out.shape == (B, S, H, D) and out.dtype == q.dtype
     assert out.stride(-1) == 1 and out.data_ptr() % 16 == 0
-    strides = (L.strides3(q.stride(0), q.stride(1), q.stride(2)),
-               L.strides3(k.stride(0), k.stride(1), k.stride(2)),
-               L.strides3(v.stride(0), v.stride(1), v.stride(2)),
-               L.strides3(out.stride(0), out.stride(2), out.stride(1)))
-    with torch.cuda.device(dev):
+    strides = (_s3(q, 0, 1, 2),
+               _s3(k, 0, 1, 2),
+               _s3(v, 0, 1, 2),
+               _s3(out, 0, 2, 1))
+    with _device(dev):
         if rows is not None:
             rc = L.lib().da_sparse_attn_fwd_rows(
                 _ptr(q), _ptr(k), _ptr(v), _ptr(out), B, H, Hkv, S, D, *strides,
@@ -142,16 +166,16 @@ def sparse_attention_delta(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *,
     if delta_out is not None:
         assert delta_out.shape == dense_sel.shape and delta_out.dtype == q.dtype
         assert delta_out.stride(-1) == 1
-        dl = L.strides3(delta_out.stride(0), delta_out.stride(2), delta_out.stride(1))
-    with torch.cuda.device(dev):
+        dl = _s3(delta_out, 0, 2, 1)
+    with _device(dev):
         rc = L.lib().da_sparse_attn_delta_fwd(
             _ptr(q), _ptr(k), _ptr(v), _ptr(out), B, H, Hkv, S, D,
-            L.strides3(q.stride(0), q.stride(1), q.stride(2)),
-            L.strides3(k.stride(0), k.stride(1), k.stride(2)),
-            L.strides3(v.stride(0), v.stride(1), v.stride(2)),
-            L.strides3(out.stride(0), out.stride(2), out.stride(1)),
+            _s3(q, 0, 1, 2),
+            _s3(k, 0, 1, 2),
+            _s3(v, 0, 1, 2),
+            _s3(out, 0, 2, 1),
             int(window), int(sink), int(q_block), float(sm_scale),
-            _ptr(dense_sel), L.strides3(dense_sel.stride(0), dense_sel.stride(2), dense_sel.stride(1)),
+            _ptr(dense_sel), _s3(dense_sel, 0, 2, 1),
             int(gamma), int(s_p), _ptr(delta_out), dl, _code(q), _stream(dev))
     L.check(rc, "da_sparse_attn_delta_fwd")
     return out
@@ -160,8 +184,18 @@ def sparse_attention_delta(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *,
 # ---------------------------------------------------------------------------
 # kernel (2)
 
+@functools.lru_cache(maxsize=256)
+def _qsparse_ws_bytes(B: int, H: int, Hkv: int, n: int, Skv: int, D: int) -> int:
+    return int(L.lib().da_qsparse_workspace_bytes(B, H, Hkv, n, Skv, D))
+
+
+@functools.lru_cache(maxsize=256)
+def _decode_ws_bytes(B: int, H: int, Hkv: int, n: int, D: int, window: int, sink: int) -> int:
+    return int(L.lib().da_decode_workspace_bytes(B, H, Hkv, n, D, window, sink))
+
+
 def qsparse_workspace(B: int, H: int, Hkv: int, n: int, Skv: int, D: int, device) -> torch.Tensor:
-    nbytes = int(L.lib().da_qsparse_workspace_bytes(B, H, Hkv, n, Skv, D))
+    nbytes = _qsparse_ws_bytes(B, H, Hkv, n, Skv, D)
     return torch.empty(max(nbytes, 16), dtype=torch.uint8, device=device)
 
 
@@ -215,15 +249,15 @@ def qsparse_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         if out is None:
             out = torch.empty((B, H, n, D), device=dev, dtype=q.dtype)
         assert out.shape == (B, H, n, D)
-        o_str = L.strides3(out.stride(0), out.stride(1), out.stride(2))
+        o_str = _s3(out, 0, 1, 2)
     else:
         assert out is not None and out.dim() == 4 and out.shape[0] == B and out.shape[2] == H
-        o_str = L.strides3(out.stride(0), out.stride(2), out.stride(1))
+        o_str = _s3(out, 0, 2, 1)
     assert out.dtype == q.dtype and out.stride(-1) == 1
     d_str = None
     if epi in (L.DA_EPI_DELTA, L.DA_EPI_DENSE) and n_anchor > 0:
         assert delta is not None and delta.shape == (B, n_anchor, H, D) and delta.dtype == q.dtype
-        d_str = L.strides3(delta.stride(0), delta.stride(2), delta.stride(1))
+        d_str = _s3(delta, 0, 2, 1)
     if n_live is not None and n > 0:
         assert epi == L.DA_EPI_OUTPUT and n_live >= 1
         if n_dev is not None:
@@ -232,26 +266,26 @@ def qsparse_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
             nb = L.lib().da_qsparse_workspace_bytes_live(B, H, Hkv, n, int(n_live), Skv, D)
             assert nb > 0, "selected-rows launch too large"
             workspace = torch.empty(nb, dtype=torch.uint8, device=dev)
-        with torch.cuda.device(dev):
+        with _device(dev):
             rc = L.lib().da_qsparse_attn_fwd_live(
                 _ptr(q), _ptr(k), _ptr(v), _ptr(q_rows), _ptr(rl), int(rl_b),
                 n, int(n_live), _ptr(n_dev), B, H, Hkv, Sq, Skv, D,
-                L.strides3(q.stride(0), q.stride(1), q.stride(2)),
-                L.strides3(k.stride(0), k.stride(1), k.stride(2)),
-                L.strides3(v.stride(0), v.stride(1), v.stride(2)),
+                _s3(q, 0, 1, 2),
+                _s3(k, 0, 1, 2),
+                _s3(v, 0, 1, 2),
                 _ptr(out), o_str, float(sm_scale), _ptr(workspace), workspace.numel(), _code(q),
                 _stream(dev))
         L.check(rc, "da_qsparse_attn_fwd_live")
         return out
     if workspace is None:
         workspace = qsparse_workspace(B, H, Hkv, n, Skv, D, dev)
-    with torch.cuda.device(dev):
+    with _device(dev):
         rc = L.lib().da_qsparse_attn_fwd(
             _ptr(q), _ptr(k), _ptr(v), _ptr(q_rows), _ptr(rl), int(rl_b),
             n, B, H, Hkv, Sq, Skv, D,
-            L.strides3(q.stride(0), q.stride(1), q.stride(2)),
-            L.strides3(k.stride(0), k.stride(1), k.stride(2)),
-            L.strides3(v.stride(0), v.stride(1), v.stride(2)),
+            _s3(q, 0, 1, 2),
+            _s3(k, 0, 1, 2),
+            _s3(v, 0, 1, 2),
             _ptr(out), o_str, int(epi), int(n_anchor), _ptr(delta), d_str,
             float(sm_scale), _ptr(workspace), workspace.numel(), _code(q), _stream(dev))
     L.check(rc, "da_qsparse_attn_fwd")
@@ -278,20 +312,20 @@ def delta_add(sparse: torch.Tensor, *, s_p: int, out: Optional[torch.Tensor] = N
     assert out.dtype == sparse.dtype and out.shape[0] == B and out.shape[2:] == (H, D)
     if delta is not None:
         n = delta.shape[1]
-        d_str = L.strides3(delta.stride(0), delta.stride(2), delta.stride(1))
+        d_str = _s3(delta, 0, 2, 1)
         ds_str = None
     else:
         assert dense_sel is not None and anchors is not None
         n = dense_sel.shape[1]
         d_str = None
-        ds_str = L.strides3(dense_sel.stride(0), dense_sel.stride(2), dense_sel.stride(1))
+        ds_str = _s3(dense_sel, 0, 2, 1)
     if anchors is not None:
         anchors = anchors.reshape(-1).to(device=dev, dtype=torch.int64).contiguous()
         assert anchors.numel() == n
-    with torch.cuda.device(dev):
+    with _device(dev):
         rc = L.lib().da_delta_add(
-            _ptr(sparse), L.strides3(sparse.stride(0), sparse.stride(2), sparse.stride(1)),
-            _ptr(out), L.strides3(out.stride(0), out.stride(2), out.stride(1)),
+            _ptr(sparse), _s3(sparse, 0, 2, 1),
+            _ptr(out), _s3(out, 0, 2, 1),
             _ptr(delta), d_str, _ptr(dense_sel), ds_str, _ptr(anchors),
             int(n), int(gamma), int(s_p), B, H, D, _code(sparse), _stream(dev))
     L.check(rc, "da_delta_add")
@@ -300,10 +334,6 @@ def delta_add(sparse: torch.Tensor, *, s_p: int, out: Optional[torch.Tensor] = N
 
 # ---------------------------------------------------------------------------
 # training path: forward with saved row log-sum-exp, and the backward
-
-def _s3(t: torch.Tensor, a: int, b: int, c: int):
-    return L.strides3(t.stride(a), t.stride(b), t.stride(c))
-
 
 def sparse_attention_lse(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, window: int,
                          sink: int, sm_scale: float, q_block: int = Q_BLOCK
@@ -317,7 +347,7 @@ def sparse_attention_lse(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, w
     q, k, v = _ready(q), _ready(k), _ready(v)
     out = torch.empty((B, S, H, D), device=dev, dtype=q.dtype)
     lse = torch.empty((B, H, S), device=dev, dtype=torch.float32)
-    with torch.cuda.device(dev):
+    with _device(dev):
         rc = L.lib().da_sparse_attn_fwd_lse(
             _ptr(q), _ptr(k), _ptr(v), _ptr(out), B, H, Hkv, S, D,
             _s3(q, 0, 1, 2), _s3(k, 0, 1, 2), _s3(v, 0, 1, 2), _s3(out, 0, 2, 1),
@@ -341,7 +371,7 @@ def rows_attention_lse(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, rows: 
     out = torch.empty((B, n, H, D), device=dev, dtype=q.dtype)
     lse = torch.empty((B, H, n), device=dev, dtype=torch.float32)
     ws = qsparse_workspace(B, H, Hkv, n, Skv, D, dev)
-    with torch.cuda.device(dev):
+    with _device(dev):
         rc = L.lib().da_qsparse_attn_fwd_lse(
             _ptr(q), _ptr(k), _ptr(v), _ptr(rows), _ptr(rows), 0, n, B, H, Hkv, Sq, Skv, D,
             _s3(q, 0, 1, 2), _s3(k, 0, 1, 2), _s3(v, 0, 1, 2), _ptr(out), _s3(out, 0, 2, 1),
@@ -375,7 +405,7 @@ def sparse_attention_bwd(q, k, v, out, dout, lse, *, window: int, sink: int, sm_
     nbytes = int(L.lib().da_sparse_attn_bwd_workspace_bytes(B, H, Hkv, S, D, int(window),
                                                             int(sink), int(q_block)))
     ws = torch.empty(max(nbytes, 16), device=dev, dtype=torch.uint8)
-    with torch.cuda.device(dev):
+    with _device(dev):
         rc = L.lib().da_sparse_attn_bwd(
             _ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(dout), _ptr(lse),
             _ptr(dq), _ptr(dk), _ptr(dv), B, H, Hkv, S, D,
@@ -405,7 +435,7 @@ def rows_attention_bwd(q, k, v, rows, out, dout, lse, *, sm_scale: float, dq=Non
     dq, dk, dv = _grads_like(q, k, dq, dk, dv)
     nbytes = int(L.lib().da_qsparse_attn_bwd_workspace_bytes(B, H, Hkv, n, Skv, D))
     ws = torch.empty(max(nbytes, 16), device=dev, dtype=torch.uint8)
-    with torch.cuda.device(dev):
+    with _device(dev):
         rc = L.lib().da_qsparse_attn_bwd(
             _ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(dout), _ptr(lse), _ptr(rows), _ptr(rows), n,
             _ptr(dq), _ptr(dk), _ptr(dv), B, H, Hkv, Sq, Skv, D,
@@ -426,7 +456,7 @@ def delta_compose_bwd(grad: torch.Tensor, *, gamma: int, s_p: int, delta_grad_sc
     n_sel = s_p // gamma + S - s_p
     dsparse = torch.empty((B, S, H, D), device=dev, dtype=grad.dtype)
     ddense = torch.empty((B, n_sel, H, D), device=dev, dtype=grad.dtype)
-    with torch.cuda.device(dev):
+    with _device(dev):
         rc = L.lib().da_delta_compose_bwd(
             _ptr(grad), _s3(grad, 0, 2, 1), _ptr(dsparse), _s3(dsparse, 0, 2, 1),
             _ptr(ddense), _s3(ddense, 0, 2, 1), B, H, S, D, int(gamma), int(s_p),
@@ -461,7 +491,7 @@ def rope_qk_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch
     cos, sin = cos.contiguous(), sin.contiguous()
     ws = [None if w is None else w.to(device=dev, dtype=q.dtype).contiguous() for w in (q_norm_w, k_norm_w)]
     cs = (ctypes.c_int64 * 2)(0 if cos.shape[0] == 1 else cos.stride(0), cos.stride(1))
-    with torch.cuda.device(dev):
+    with _device(dev):
         rc = L.lib().da_rope_qk_append(
             _ptr(q), _s3(q, 0, 1, 2), Hq, _ptr(k), _s3(k, 0, 1, 2), Hkv, _ptr(v), _s3(v, 0, 1, 2),
             B, D, _ptr(cos), _ptr(sin), cs, _ptr(ws[0]), _ptr(ws[1]), float(eps),
@@ -495,11 +525,11 @@ def rope_qk(q: Optional[torch.Tensor], k: Optional[torch.Tensor], cos: torch.Ten
             assert t.stride(-1) == 1 and t.data_ptr() % 16 == 0, "rope_qk works in place on row-contiguous tensors"
     ws = [None if w is None else w.to(device=dev, dtype=x.dtype).contiguous() for w in (q_norm_w, k_norm_w)]
     cs = (ctypes.c_int64 * 2)(0 if cos.shape[0] == 1 else cos.stride(0), cos.stride(1))
-    with torch.cuda.device(dev):
+    with _device(dev):
         rc = L.lib().da_rope_qk(
-            _ptr(q), None if q is None else L.strides3(q.stride(0), q.stride(1), q.stride(2)),
+            _ptr(q), None if q is None else _s3(q, 0, 1, 2),
             0 if q is None else q.shape[2],
-            _ptr(k), None if k is None else L.strides3(k.stride(0), k.stride(1), k.stride(2)),
+            _ptr(k), None if k is None else _s3(k, 0, 1, 2),
             0 if k is None else k.shape[2],
             B, S, D, _ptr(cos), _ptr(sin), cs, _ptr(ws[0]), _ptr(ws[1]), float(eps),
             _code(x), _stream(dev))
@@ -534,13 +564,13 @@ def decode_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, windo
         out = torch.empty((B, H, 1, D), device=dev, dtype=q.dtype)
     assert out.shape == (B, H, 1, D) and out.stride(-1) == 1 and out.data_ptr() % 16 == 0
     w, sk = max(int(window), 0), max(int(sink), 0)
-    nbytes = int(L.lib().da_decode_workspace_bytes(B, H, Hkv, n, D, w, sk))
+    nbytes = _decode_ws_bytes(B, H, Hkv, n, D, w, sk)
     ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev)
-    strides = (L.strides3(q.stride(0), q.stride(1), q.stride(2)),
-               L.strides3(k.stride(0), k.stride(1), k.stride(2)),
-               L.strides3(v.stride(0), v.stride(1), v.stride(2)),
-               L.strides3(out.stride(0), out.stride(1), out.stride(2)))
-    with torch.cuda.device(dev):
+    strides = (_s3(q, 0, 1, 2),
+               _s3(k, 0, 1, 2),
+               _s3(v, 0, 1, 2),
+               _s3(out, 0, 1, 2))
+    with _device(dev):
         if n_keys is None:
             assert add is None, "add= goes with a device key count"
             rc = L.lib().da_decode_attn_fwd(
@@ -554,7 +584,7 @@ def decode_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, windo
             rc = L.lib().da_decode_attn_fwd_dev(
                 _ptr(q), _ptr(k), _ptr(v), _ptr(out), B, H, Hkv, _ptr(n_keys), n, D, *strides,
                 w, sk, float(sm_scale), _ptr(add),
-                None if add is None else L.strides3(add.stride(0), add.stride(1), add.stride(2)),
+                None if add is None else _s3(add, 0, 1, 2),
                 _ptr(ws), nbytes, _code(q), _stream(dev))
     L.check(rc, "da_decode_attn_fwd" if n_keys is None else "da_decode_attn_fwd_dev")
     return out
@@ -598,7 +628,7 @@ def add_rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, *,
         _, rs = _rows2d(residual)
         h = torch.empty_like(x) if residual_out is None else residual_out
         _, hs = _rows2d(h)
-    with torch.cuda.device(dev):
+    with _device(dev):
         rc = L.lib().da_add_rmsnorm(_ptr(x), xs, _ptr(residual), rs, _ptr(h), hs, _ptr(out), ys,
                                     _ptr(w), rows, n, float(eps), _code(x), _stream(dev))
     L.check(rc, "da_add_rmsnorm")
@@ -614,7 +644,7 @@ def swiglu(gate: torch.Tensor, up: torch.Tensor, out: Optional[torch.Tensor] = N
     if out is None:
         out = torch.empty_like(gate)
     _, os_ = _rows2d(out)
-    with torch.cuda.device(dev):
+    with _device(dev):
         rc = L.lib().da_swiglu(_ptr(gate), gs, _ptr(up), us, _ptr(out), os_, rows, gate.shape[-1],
                                _code(gate), _stream(dev))
     L.check(rc, "da_swiglu")
@@ -658,7 +688,7 @@ def anchor_delta_cos(a: torch.Tensor, *, sparse: Optional[torch.Tensor] = None,
         if rows is not None:
             rows = rows.to(device=dev, dtype=torch.int64).contiguous()
             assert rows.numel() == n, (rows.numel(), n)
-    with torch.cuda.device(dev):
+    with _device(dev):
         rc = L.lib().da_anchor_delta_cos(
             _ptr(a), L.I64x3(*a.stride()[:3]), _ptr(sparse), s_str, _ptr(rows), n_rows,
             B, n, H, D, _ptr(cos), _ptr(hist), int(hist_bins),
@@ -693,7 +723,7 @@ def adapt_chunk_step(dense: torch.Tensor, sparse: torch.Tensor, rows: torch.Tens
     assert trigger in ("absolute", "relative"), trigger
     if rows_next is not None:
         assert rows_next.dtype == torch.int64 and rows_next.is_contiguous() and rows_next.numel() == max_n
-    with torch.cuda.device(dev):
+    with _device(dev):
         rc = L.lib().da_adapt_chunk_step(
             _ptr(dense), L.I64x3(*dense.stride()[:3]), _ptr(sparse), L.I64x3(*sparse.stride()[:3]),
             int(sparse.shape[1]), _ptr(rows), B, H, D, max_n, _ptr(state), _ptr(cos_work), int(chunk),
@@ -736,13 +766,13 @@ def adapt_layer(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Te
     log_min = torch.empty(n_log, dtype=torch.float32, device=dev)
     log_gamma = torch.empty(n_log, dtype=torch.int32, device=dev)
     log_n = torch.empty(n_log, dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
+    with _device(dev):
         rc = L.lib().da_adapt_layer_fwd(
             _ptr(q), _ptr(k), _ptr(v), _ptr(out), B, H, Hkv, S, D,
-            L.strides3(q.stride(0), q.stride(1), q.stride(2)),
-            L.strides3(k.stride(0), k.stride(1), k.stride(2)),
-            L.strides3(v.stride(0), v.stride(1), v.stride(2)),
-            L.strides3(out.stride(0), out.stride(2), out.stride(1)),
+            _s3(q, 0, 1, 2),
+            _s3(k, 0, 1, 2),
+            _s3(v, 0, 1, 2),
+            _s3(out, 0, 2, 1),
             int(window), int(sink), int(q_block), float(sm_scale), int(s_p), int(adapt_chunk),
             int(gamma0), int(gamma_min), int(gamma_max), 0 if trigger == "absolute" else 1,
             float(threshold), float(margin), float(k_sd), _ptr(log_mean), _ptr(log_min),
@@ -769,6 +799,18 @@ def selected_rows(s: int, gamma: int, device: str) -> torch.Tensor:
     s_p = max(s_p, 0)
     return torch.cat([torch.arange(0, s_p, gamma, dtype=torch.int64),
                       torch.arange(s_p, s, dtype=torch.int64)]).to(device)
+
+
+@functools.lru_cache(maxsize=64)
+def _selected_rows_of_stream(s: int, gamma: int, device: str, stream: int) -> torch.Tensor:
+    return selected_rows.__wrapped__(s, gamma, device)
+
+
+def selected_rows_here(s: int, gamma: int, device: torch.device) -> torch.Tensor:
+    """selected_rows in a tensor of torch's current stream, kept per size and
+    stream: a caller's every use of it is then ordered with its memory's reuse
+    (building it takes a blocking host-to-device copy, about 25 us)."""
+    return _selected_rows_of_stream(s, gamma, str(device), _stream(device))
 
 
 def delta_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, gamma: int,

@@ -44,20 +44,18 @@ class _DeltaAttention(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, gamma, window, sink, scaling, detach_delta, delta_grad_scale):
         b, h, s, d = q.shape
-        idx, tail, s_p = anchor_layout(s, gamma)
-        if s_p <= 0:
-            # no anchors: every row is a dense tail row
-            idx, tail, s_p = idx[:0], torch.arange(0, s), 0
-        sel = torch.cat((idx, tail)).to(q.device)
+        # s_p <= 0: no anchors, every row is a dense tail row
+        _, s_p, n = ops.anchor_layout(s, gamma)
+        s_p = max(s_p, 0)
+        sel = ops.selected_rows_here(s, gamma, q.device)
         sparse, lse_s = ops.sparse_attention_lse(q, k, v, window=window, sink=sink,
                                                  sm_scale=scaling, q_block=Q_BLOCK)
         dense_sel, lse_d = ops.rows_attention_lse(q, k, v, sel, scaling)
-        n = idx.numel()
         out = torch.empty((b, s, h, d), device=q.device, dtype=q.dtype)
         if s_p > 0:
             # delta = rnd(dense_anchor - sparse[idx]); out = rnd(sparse + delta)
             ops.delta_add(sparse, s_p=s_p, out=out[:, :s_p], dense_sel=dense_sel[:, :n],
-                          anchors=idx.to(q.device), gamma=gamma)
+                          anchors=sel[:n], gamma=gamma)
         out[:, s_p:] = dense_sel[:, n:]
         ctx.save_for_backward(q, k, v, sel, sparse, lse_s, dense_sel, lse_d)
         ctx.cfg = (gamma, window, sink, scaling, detach_delta, delta_grad_scale, s_p)
