@@ -113,8 +113,9 @@ template <> struct Rescale<_Float16> {
   static constexpr float lsum = 32768.0f;           // 2^15
 };
 
-// MODE_FUSED is MODE_SPARSE with the delta broadcast-add in its epilogue.
-enum { MODE_SPARSE = 0, MODE_QSPARSE = 1, MODE_FUSED = 2 };
+// MODE_FUSED is MODE_SPARSE with the delta broadcast-add in its epilogue,
+// MODE_STREAM is MODE_QSPARSE with non-temporal K/V loads (see streams_kv).
+enum { MODE_SPARSE = 0, MODE_QSPARSE = 1, MODE_FUSED = 2, MODE_STREAM = 3 };
 
 struct AttnArgs {
   const void* q;
@@ -155,6 +156,7 @@ struct AttnArgs {
   // [item][ws_rows][D]: each row's O / l, float when part_f32, else elements
   void* part_o;
   int part_f32;
+  int ref_first;    // query-sparse mode: splits take the row max of the list's first tile
   float* part_ml;   // [item][2][ws_rows]  (running max, row sum)
   int ws_rows;      // workspace rows per item: min(bm, n_rows * G) (a tile's valid rows)
   // MODE_FUSED: dense anchor rows [B, n_anchor, Hq, D] (strides batch, head,
@@ -287,7 +289,8 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
   const int lg = lane >> 5;
 
   // ---- work item (XCD-aware: each XCD walks a contiguous range) ----
-  constexpr bool KSPARSE = MODE != MODE_QSPARSE;
+  constexpr bool KSPARSE = MODE == MODE_SPARSE || MODE == MODE_FUSED;
+  constexpr bool NT = MODE == MODE_STREAM;
   const bool live = !KSPARSE && a.n_rows_dev;
   int w;
   int mt, split = 0, bh, hs = 0;
@@ -495,20 +498,20 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
     const __amdgpu_buffer_rsrc_t rk = tile_rsrc(kbase, kend, krow_b, t);
 #pragma unroll
     for (int c = 0; c < NDMA; ++c)
-      dma16(rk, (DA_LDS void*)(&smem[slot][0][(c * NWAVE + wave) * 1024]), koff[c]);
+      dma16<NT>(rk, (DA_LDS void*)(&smem[slot][0][(c * NWAVE + wave) * 1024]), koff[c]);
   };
   // key tile t into the V buffer of stage 1 (free until V(1) is issued)
   auto issue_ref = [&](int t) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t rk = tile_rsrc(kbase, kend, krow_b, t);
 #pragma unroll
     for (int c = 0; c < NDMA; ++c)
-      dma16(rk, (DA_LDS void*)(&smem[1][1][(c * NWAVE + wave) * 1024]), koff[c]);
+      dma16<NT>(rk, (DA_LDS void*)(&smem[1][1][(c * NWAVE + wave) * 1024]), koff[c]);
   };
   auto issue_v = [&](int t, int slot) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t rv = tile_rsrc(vbase, vend, vrow_b, t);
 #pragma unroll
     for (int c = 0; c < NDMA; ++c)
-      dma16(rv, (DA_LDS void*)(&smem[slot][1][(c * NWAVE + wave) * 1024]), voff[c]);
+      dma16<NT>(rv, (DA_LDS void*)(&smem[slot][1][(c * NWAVE + wave) * 1024]), voff[c]);
   };
 
   // ---- LDS read offsets ----
@@ -878,7 +881,7 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
       // composition subtracts (with a max per split the composed output of a
       // 1531-token layer was 6 % further from 64-bit arithmetic). One more
       // score product per item, no extra wait.
-      const bool ref = !KSPARSE && a.part_f32 && t_off > 0;
+      const bool ref = !KSPARSE && a.ref_first && t_off > 0;
       if (ref) issue_ref(-t_off);
       wait_vmcnt<0>();
       __syncthreads();
@@ -1504,18 +1507,59 @@ static QsparsePlan plan_rows_live(int B, int Hq, int Hkv, int n, int n_live, int
 }
 
 // One decode row per batch at the end of the cache: its list is the sink
-// tiles plus the window tiles (all tiles without a window); ~512 items.
-static QsparsePlan plan_decode(int B, int Hq, int Hkv, int n_keys, int D, int window, int sink) {
-  const int64_t all = (n_keys + BN - 1) / BN;
-  int64_t vis = all;
-  if (window > 0) vis = min(all, (int64_t)(min(sink, n_keys) + BN - 1) / BN + (window + BN - 1) / BN + 1);
+// tiles plus the window tiles (all tiles without a window). The fewest full
+// rounds of the resident workgroups whose items hold at most 40 tiles: a round
+// that starts half empty costs a whole item's time, and longer items end
+// unevenly over the memory channels (7 x 32 heads, 30000 keys: 203 us at 560
+// items of 47 tiles, 160 us at 1008 of 27; 32 x 32 heads, 20000 keys 485 us at
+// 512 items, 445 us at 2048; head_dim 256, 4 kv heads, 20000 keys, on its 256
+// slots: 31.9 -> 25.0 us). The partials, a few rows an item, are fp32. A plan
+// past the static scratch of da_decode_attn_fwd_dev_noalloc gives way to one
+// of about DA_DECODE_ITEMS items with 16-bit partials.
+static QsparsePlan plan_decode_short(int B, int Hq, int Hkv, int64_t vis, int D) {
   return plan_qsparse(B, Hq, Hkv, 1, vis, D, DA_DECODE_ITEMS, 1, bm_of(1));
+}
+
+static int64_t decode_tiles(int n_keys, int window, int sink) {
+  const int64_t all = (n_keys + BN - 1) / BN;
+  if (window <= 0) return all;
+  return min(all, (int64_t)(min(sink, n_keys) + BN - 1) / BN + (window + BN - 1) / BN + 1);
+}
+
+static QsparsePlan plan_decode(int B, int Hq, int Hkv, int n_keys, int D, int window, int sink) {
+  const int64_t vis = decode_tiles(n_keys, window, sink);
+  const QsparsePlan old = plan_decode_short(B, Hq, Hkv, vis, D);
+  const int64_t tiles = (int64_t)B * Hkv * old.n_mtiles, slots = resident_slots(D);
+  if (old.n_items <= 0 || tiles > 64 * slots) return old;
+  int64_t splits = 0;
+  for (int64_t r = 1; splits < vis; ++r) {
+    splits = min(slots * r / tiles, vis);
+    if (splits > 0 && (vis + splits - 1) / splits <= 40) break;
+  }
+  if (tiles * splits > (1 << 24)) return old;
+  const QsparsePlan p = plan_qsparse(B, Hq, Hkv, 1, vis, D, (int)(tiles * splits), 1, bm_of(1),
+                                     0x7fffffff, true);
+  if (p.n_items <= 0 || (p.ws_bytes > old.ws_bytes && p.ws_bytes > DA_DECODE_SCRATCH_BYTES)) return old;
+  return p;
+}
+
+// Whether a selected-rows or decode launch takes non-temporal K/V loads: each
+// key tile is read by one workgroup (one row tile per kv head), and the caches
+// could not hold the keys for the next pass anyway (more than the 256 MB of
+// the memory-side cache). A dense row of 32 heads over 131072 keys 106 -> 89
+// us (5.1 -> 6.0 TB/s; a plain read loop reaches 6.1 TB/s, 6.9 non-temporal),
+// 16 x 40 heads over 6007 keys 80 -> 71 us, 32 x 32 heads over 20000 keys 445
+// -> 400 us; where a repeated pass finds its keys in that cache (2 x 32 heads,
+// 20000 keys, 164 MB) non-temporal loads are slower, 35 -> 39 us.
+static bool streams_kv(const QsparsePlan& p, int B, int Hkv, int D) {
+  return p.n_mtiles == 1 && (int64_t)B * Hkv * p.vis * (BN * 4) * D > (int64_t)256 << 20;
 }
 
 template <typename T, int D, int MODE>
 static void launch_attn(const AttnArgs& a, hipStream_t stream) {
   const int grid = (a.n_items + 7) / 8 * 8;
-  constexpr bool has_rg2 = D == 128 && (MODE != MODE_QSPARSE || DA_RG_ROWS == 2);
+  constexpr bool has_rg2 =
+      D == 128 && (MODE == MODE_SPARSE || MODE == MODE_FUSED || DA_RG_ROWS == 2);
   if constexpr (has_rg2) {
     if (a.bm == bm_of(2)) {
       hipLaunchKernelGGL((attn_fwd_kernel<T, D, MODE, 2>), dim3(grid), dim3(NTHR), 0, stream, a);
@@ -1756,6 +1800,7 @@ static int run_qsparse(const QsparsePlan& p, const void* q, const void* k, const
   a.window = window; a.sink = sink;
   a.vis = (int)p.vis; a.slots = (int)resident_slots(D);
   a.part_o = workspace; a.part_f32 = p.f32;
+  a.ref_first = p.f32 && row_last;
   a.part_ml = (float*)((char*)workspace +
                        (size_t)p.n_items * p.ws_rows * D * (p.f32 ? sizeof(float) : sizeof(uint16_t)));
   a.ws_rows = p.ws_rows;
@@ -1794,7 +1839,8 @@ static int run_qsparse(const QsparsePlan& p, const void* q, const void* k, const
 
   hipStream_t s = (hipStream_t)stream;
   (void)hipGetLastError();
-  dispatch_attn<MODE_QSPARSE>(a, D, dtype, s);
+  if (streams_kv(p, B, Hkv, D)) dispatch_attn<MODE_STREAM>(a, D, dtype, s);
+  else dispatch_attn<MODE_QSPARSE>(a, D, dtype, s);
   const int n_tiles = B * Hkv * p.n_mtiles * m.wgs;
   if (dtype == DA_BF16) {
     if (D == 128) launch_merge<__bf16, 128>(m, n_tiles, p.f32, s);
@@ -2010,7 +2056,10 @@ extern "C" int da_decode_attn_fwd_dev_noalloc(const void* q, const void* k, cons
   int rc;
   if ((rc = check_common(B, Hq, Hkv, D, dtype)) != DA_OK) return rc;
   if (max_keys < 1 || window < 0 || sink < 0) return DA_ERR_INVALID_ARG;
-  const size_t need = plan_decode(B, Hq, Hkv, max_keys, D, window, sink).ws_bytes;
+  // (the sizes the scratch serves are those of the short plan, which
+  // plan_decode falls back to)
+  const size_t need =
+      plan_decode_short(B, Hq, Hkv, decode_tiles(max_keys, window, sink), D).ws_bytes;
   if (need == 0 || need > DA_DECODE_SCRATCH_BYTES) return DA_ERR_SCRATCH;
   void* ws = nullptr;
   if ((rc = scratch_address(&ws)) != DA_OK) return rc;

@@ -128,8 +128,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, ui
 
 // 16 bytes per lane from global memory straight into LDS: lane i of the wave
 // writes LDS bytes [lds + 16 i, lds + 16 i + 16). `lds` must be wave-uniform.
+// NT: non-temporal (data no later pass finds in a cache).
+template <bool NT = false>
 __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, DA_LDS void* lds, uint32_t voff) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds, 16, voff, 0, 0, 0);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds, 16, voff, 0, 0, NT ? 2 : 0);
 }
 
 // Division by a divisor fixed for a launch (d >= 1) of dividends in
