@@ -32,12 +32,15 @@
 //     dK^T += Q^T dS from transposed LDS reads. Sink keys are seen by every
 //     later row, so their row range is cut into chunks like any other; each
 //     chunk writes fp32 partials that dkdv_reduce_kernel sums per key.
+//   * dkdv_pipe_kernel: the same for key-sparse attention at head_dim 128, as
+//     one static schedule over a ring of (row step, head) units.
 // Every MFMA is v_mfma_f32_32x32x16 (bf16 or fp16 operands, fp32 accumulate).
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
 
 #include "device_common.h"
+#include "agpr_tiles.h"
 #include "capi_common.h"
 
 namespace da {
@@ -483,6 +486,54 @@ __global__ __launch_bounds__(RED) void dq_reduce_kernel(BwdArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// Writes one dkdv item's results (element j of tile dt: dim 32 dt + 8 (j / 4)
+// + 4 lg + j % 4 of key `key`, row `row` of its block).
+template <typename T, int D>
+__device__ __forceinline__ void dkdv_store(const BwdArgs& a, const f32x16 (&adk)[D / 32],
+                                           const f32x16 (&adv)[D / 32], int b, int hk, int bh,
+                                           int blk, int item, int key, int row, int lg) {
+  constexpr int NDT = D / 32;
+  const size_t esz = sizeof(T);
+  // A block whose rows are one item writes its dK (scaled by sm_scale) and
+  // dV directly, as the reduce would from a single partial (the same bits);
+  // a block of several items writes partials [2][KT][D] for the reduce.
+  if ((blk < a.nsb ? a.ncs : a.nco) == 1) {
+    if (key >= a.n_kv) return;
+    u32x2* ok = (u32x2*)((char*)a.dk + ((int64_t)b * a.dks_b + (int64_t)hk * a.dks_h + (int64_t)key * a.dks_s) * esz);
+    u32x2* ov = (u32x2*)((char*)a.dv + ((int64_t)b * a.dvs_b + (int64_t)hk * a.dvs_h + (int64_t)key * a.dvs_s) * esz);
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int jq = 0; jq < 4; ++jq) {
+        const int d4 = (32 * dt + 8 * jq + 4 * lg) / 4;
+        const u32x2 pk0 = a.accumulate ? ok[d4] : (u32x2){0, 0};
+        const u32x2 pv0 = a.accumulate ? ov[d4] : (u32x2){0, 0};
+        u32x2 nk, nv;
+        nk[0] = acc_pack<T>(pk0[0], adk[dt][4 * jq] * a.sm_scale, adk[dt][4 * jq + 1] * a.sm_scale, a.accumulate);
+        nk[1] = acc_pack<T>(pk0[1], adk[dt][4 * jq + 2] * a.sm_scale, adk[dt][4 * jq + 3] * a.sm_scale, a.accumulate);
+        nv[0] = acc_pack<T>(pv0[0], adv[dt][4 * jq], adv[dt][4 * jq + 1], a.accumulate);
+        nv[1] = acc_pack<T>(pv0[1], adv[dt][4 * jq + 2], adv[dt][4 * jq + 3], a.accumulate);
+        ok[d4] = nk;
+        ov[d4] = nv;
+      }
+    return;
+  }
+  // (those items come first in a (batch, kv head)'s item order: every item
+  // when the window blocks are cut too, else the sink blocks' items)
+  float* pk = a.kv_part + ((int64_t)bh * a.part_per_bh + item) * 2 * KT * D + (int64_t)row * D;
+  float* pv = pk + (int64_t)KT * D;
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+    for (int jq = 0; jq < 4; ++jq) {
+      const int d = 32 * dt + 8 * jq + 4 * lg;
+      *(f32x4*)(pk + d) = (f32x4){adk[dt][4 * jq] * a.sm_scale, adk[dt][4 * jq + 1] * a.sm_scale,
+                                  adk[dt][4 * jq + 2] * a.sm_scale, adk[dt][4 * jq + 3] * a.sm_scale};
+      *(f32x4*)(pv + d) = (f32x4){adv[dt][4 * jq], adv[dt][4 * jq + 1],
+                                  adv[dt][4 * jq + 2], adv[dt][4 * jq + 3]};
+    }
+}
+
 template <typename T, int D, bool ROWS>
 __global__ __launch_bounds__(NTHR, 1) void dkdv_kernel(BwdArgs a) {
   using E = Elt<T>;
@@ -845,44 +896,323 @@ __global__ __launch_bounds__(NTHR, 1) void dkdv_kernel(BwdArgs a) {
     }
   }
 
-  // A block whose rows are one item writes its dK (scaled by sm_scale) and
-  // dV directly, as the reduce would from a single partial (the same bits);
-  // a block of several items writes partials [2][KT][D] for the reduce.
-  if ((blk < a.nsb ? a.ncs : a.nco) == 1) {
-    if (key >= a.n_kv) return;
-    u32x2* ok = (u32x2*)((char*)a.dk + ((int64_t)b * a.dks_b + (int64_t)hk * a.dks_h + (int64_t)key * a.dks_s) * esz);
-    u32x2* ov = (u32x2*)((char*)a.dv + ((int64_t)b * a.dvs_b + (int64_t)hk * a.dvs_h + (int64_t)key * a.dvs_s) * esz);
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-      for (int jq = 0; jq < 4; ++jq) {
-        const int d4 = (32 * dt + 8 * jq + 4 * lg) / 4;
-        const u32x2 pk0 = a.accumulate ? ok[d4] : (u32x2){0, 0};
-        const u32x2 pv0 = a.accumulate ? ov[d4] : (u32x2){0, 0};
-        u32x2 nk, nv;
-        nk[0] = acc_pack<T>(pk0[0], adk[dt][4 * jq] * a.sm_scale, adk[dt][4 * jq + 1] * a.sm_scale, a.accumulate);
-        nk[1] = acc_pack<T>(pk0[1], adk[dt][4 * jq + 2] * a.sm_scale, adk[dt][4 * jq + 3] * a.sm_scale, a.accumulate);
-        nv[0] = acc_pack<T>(pv0[0], adv[dt][4 * jq], adv[dt][4 * jq + 1], a.accumulate);
-        nv[1] = acc_pack<T>(pv0[1], adv[dt][4 * jq + 2], adv[dt][4 * jq + 3], a.accumulate);
-        ok[d4] = nk;
-        ov[d4] = nv;
-      }
-    return;
+  dkdv_store<T, D>(a, adk, adv, b, hk, bh, blk, item, key, wave * 32 + ln, lg);
+}
+
+// dkdv_kernel for the key-sparse attention at head_dim 128, as one static
+// schedule. With one wave per SIMD nothing hides a fragment read or the
+// softmax chain: the compiler's order of dkdv_kernel waits for LDS 36 times
+// per head and took about 2900 cycles for its 32 MFMAs (1024 cycles). Here
+//  * the (32-row step, query head) pairs of the item, heads innermost, are one
+//    stream of units through a ring of eight LDS slots filled by DMA (Q and dO
+//    rows, row statistics); every second unit one barrier frees two slots,
+//    whose next units are issued in the following iteration, one operation a
+//    slot, and have three units' time to land;
+//  * unit i's iteration holds, in 32 slots of one MFMA each, the score
+//    products S, dP of unit i + 1 (slots 0-15) with the softmax of unit i
+//    under them, then dV, dK of unit i (slots 16-31); fragment reads run four
+//    slots ahead;
+//  * dV and dK live in the reserved AGPR tiles (agpr_tiles.h: dV 0-3, dK 4-7),
+//    the K and V fragments in the AGPRs below them.
+// Rows past the chunk end read as zero and are masked like rows out of a key's
+// window.
+// 32 heads / 8 at 32768 rows, window 2048: both key-sparse backward kernels
+// 4.59 -> 4.16 ms (this one about 2.73 -> 2.3); 8 / 8 heads at 16384 rows 858
+// -> 580 us. On copies that drop work: no DMA -350 us, no transposed reads
+// -190, no exponentials -150; what is left, 1.7 ms, is the MFMA issue rate of
+// one wave per SIMD (about 50 cycles each). Issued between the iterations
+// instead of one a slot, the DMAs cost 160 us; plain row order instead of the
+// cyclic one 65 us.
+template <typename T>
+__global__ __launch_bounds__(NTHR, 1) void dkdv_pipe_kernel(BwdArgs a) {
+  using E = Elt<T>;
+  constexpr int D = 128, NDS = D / 16, NDT = D / 32, DCH = D / 8, RB = 2 * D;
+  constexpr int TB = RT * RB;
+  constexpr int NSLOT = 8, NDMA = TB / (NTHR * 16);     // ring slots; DMAs per tile and thread
+  constexpr int UNIT_VM = 2 * NDMA + 2;                 // vector memory operations per unit and wave
+  static_assert(NDS == 8 && NDT == 4, "32 MFMA slots");
+  // [slot][Q, dO]: the tile, then [wave][64] floats of its row statistics (lse
+  // with Q, rowsum(dO * O) with dO; 32 rows, the upper halves unused)
+  constexpr int TS = TB + NWAVE * 256;
+  __shared__ __attribute__((aligned(1024))) char smem[NSLOT][2][TS];
+  const size_t esz = sizeof(T);
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ln = lane & 31, lg = lane >> 5;
+  const int per = (int)(gridDim.x >> 3);
+  const int wi = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if (wi >= a.B * a.Hkv * a.items_per_bh) return;
+  const int item = wi % a.items_per_bh;
+  const int bh = wi / a.items_per_bh;
+  const int hk = bh % a.Hkv, b = bh / a.Hkv;
+  int blk, c;
+  if (item < a.nsb * a.ncs) {
+    blk = item / a.ncs;
+    c = item % a.ncs;
+  } else {
+    const int r = item - a.nsb * a.ncs;
+    blk = a.nsb + r / a.nco;
+    c = r % a.nco;
   }
-  // (those items come first in a (batch, kv head)'s item order: every item
-  // when the window blocks are cut too, else the sink blocks' items)
-  float* pk = a.kv_part + ((int64_t)bh * a.part_per_bh + item) * 2 * KT * D + (int64_t)(wave * 32 + ln) * D;
-  float* pv = pk + (int64_t)KT * D;
+  const int k0 = blk * KT;
+  const uint32_t lds_w = (uint32_t)(uintptr_t)(DA_LDS char*)&smem[0][0][0];
+  const int kw = k0 + (wave << 5);          // this wave's first key
+  const int key = kw + ln;
+
+  // First row past the window of a key (its rows are key .. row_hi - 1), and
+  // the rows of this item
+  auto row_hi = [&](int kk) -> int {
+    const int tq = kk + a.window - a.q_block;
+    return tq < 0 ? 0 : (tq / a.q_block + 1) * a.q_block;
+  };
+  const int p_end = k0 < a.sink ? a.n_rows - 1
+                                : min(a.n_rows, row_hi(min(k0 + KT - 1, a.n_kv - 1))) - 1;
+  const int c_start = k0 + c * a.rpc;
+  const int c_end = min(p_end, c_start + a.rpc - 1);
+  const int rhi = min(c_end + 1, key < a.sink ? 0x7fffffff : row_hi(key));
+  // rows below see every key of the wave that is not above them
+  const int rhi_w = min(c_end + 1, kw + 31 < a.sink ? 0x7fffffff : row_hi(kw));
+  const int n_steps = c_end >= c_start ? (c_end - c_start) / RT + 1 : 0;
+  const int n = n_steps * a.G;
+  // The row steps are walked cyclically from the one whose number (row / 32)
+  // is a multiple of n_steps: key blocks of the same length that run beside
+  // each other on an XCD, each starting 128 rows after the last, then read the
+  // same rows at the same time, and the rows come from L2 (in plain order the
+  // 32 blocks of an XCD read 12 MB of rows apart).
+  const int r_first = n_steps > 0 ? c_start + (n_steps - 1 - (c_start / RT + n_steps - 1) % n_steps) * RT : 0;
+
+  // ---- unit stream: DMA of unit u (row step, head) into slot u % 8, issued
+  //      in order ----
+  const uint32_t qrow_b = (uint32_t)(a.qs_s * (int64_t)esz), grow_b = (uint32_t)(a.gs_s * (int64_t)esz);
+  const char* qb0 = (const char*)a.q + ((int64_t)b * a.qs_b + (int64_t)hk * a.G * a.qs_h) * esz;
+  const char* gb0 = (const char*)a.dout + ((int64_t)b * a.gs_b + (int64_t)hk * a.G * a.gs_h) * esz;
+  const int64_t st0 = ((int64_t)b * a.Hq + (int64_t)hk * a.G) * a.n_rows;
+  uint32_t qoff[NDMA], goff[NDMA];
 #pragma unroll
-  for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-    for (int jq = 0; jq < 4; ++jq) {
-      const int d = 32 * dt + 8 * jq + 4 * lg;
-      *(f32x4*)(pk + d) = (f32x4){adk[dt][4 * jq] * a.sm_scale, adk[dt][4 * jq + 1] * a.sm_scale,
-                                  adk[dt][4 * jq + 2] * a.sm_scale, adk[dt][4 * jq + 3] * a.sm_scale};
-      *(f32x4*)(pv + d) = (f32x4){adv[dt][4 * jq], adv[dt][4 * jq + 1],
-                                  adv[dt][4 * jq + 2], adv[dt][4 * jq + 3]};
+  for (int cc = 0; cc < NDMA; ++cc) {
+    const int row = ((cc * NWAVE + wave) * 64 + lane) / DCH, pc = lane % DCH;
+    const uint32_t chunk = (uint32_t)((pc ^ swz<D>(row)) * 16);
+    qoff[cc] = (uint32_t)row * qrow_b + chunk;
+    goff[cc] = (uint32_t)row * grow_b + chunk;
+  }
+  const uint32_t soff = lane < RT ? (uint32_t)lane * 4 : 0xfffffff0u;
+  int u_next = 0, u_g = 0, u_r0 = r_first;
+  const char* u_q = qb0 + (int64_t)r_first * a.qs_s * esz;
+  const char* u_d = gb0 + (int64_t)r_first * a.gs_s * esz;
+  int64_t u_s = st0 + r_first;
+  u32x4 rq, rg, rl, rd;
+  uint32_t u_lds = 0;
+  // the next unit's resources (empty past the last unit: every unit slot is
+  // issued, so that the counts of operations in flight never vary)
+  auto next_unit = [&]() __attribute__((always_inline)) {
+    const uint32_t nrow = u_next < n ? (uint32_t)min(RT, c_end - u_r0 + 1) : 0u;
+    rq = rsrc_words(u_q, nrow * qrow_b);
+    rg = rsrc_words(u_d, nrow * grow_b);
+    rl = rsrc_words(a.lse + u_s, nrow * 4);
+    rd = rsrc_words(a.dvec + u_s, nrow * 4);
+    u_lds = lds_w + (uint32_t)(u_next & (NSLOT - 1)) * (2 * TS);
+    ++u_next;
+    u_q += a.qs_h * (int64_t)esz;
+    u_d += a.gs_h * (int64_t)esz;
+    u_s += a.n_rows;
+    if (++u_g == a.G) {
+      u_g = 0;
+      u_r0 = u_r0 + RT <= c_end ? u_r0 + RT : c_start;
+      u_q = qb0 + (int64_t)u_r0 * a.qs_s * esz;
+      u_d = gb0 + (int64_t)u_r0 * a.gs_s * esz;
+      u_s = st0 + u_r0;
     }
+  };
+  // operation k of the unit's UNIT_VM
+  auto issue_op = [&](auto k_c) __attribute__((always_inline)) {
+    constexpr int k = decltype(k_c)::value;
+    if constexpr (k < NDMA) dma16_untracked(rq, u_lds + wave * 1024 + k * (NWAVE * 1024), qoff[k]);
+    else if constexpr (k < 2 * NDMA) dma16_untracked(rg, u_lds + TS + wave * 1024 + (k - NDMA) * (NWAVE * 1024), goff[k - NDMA]);
+    else if constexpr (k == 2 * NDMA) dma4_untracked(rl, u_lds + TB + wave * 256, soff);
+    else dma4_untracked(rd, u_lds + TS + TB + wave * 256, soff);
+  };
+
+  // K^T and V^T fragments of this lane's key (B operands, in AGPRs)
+  u32x4 kf[NDS], vf[NDS];
+  {
+    const bool in = key < a.n_kv;
+    const char* kp = (const char*)a.k + ((int64_t)b * a.ks_b + (int64_t)hk * a.ks_h + (int64_t)(in ? key : 0) * a.ks_s) * esz;
+    const char* vp = (const char*)a.v + ((int64_t)b * a.vs_b + (int64_t)hk * a.vs_h + (int64_t)(in ? key : 0) * a.vs_s) * esz;
+#pragma unroll
+    for (int ds = 0; ds < NDS; ++ds) {
+      kf[ds] = *(const u32x4*)(kp + (16 * ds + 8 * lg) * esz);
+      vf[ds] = *(const u32x4*)(vp + (16 * ds + 8 * lg) * esz);
+    }
+  }
+  for (int u = 0; u < NSLOT - 2; ++u) {
+    next_unit();
+    StaticFor<0, UNIT_VM>::run([&](auto k_c) __attribute__((always_inline)) { issue_op(k_c); });
+  }
+  ot_pad();
+  StaticFor<0, 2 * NDT>::run([&](auto i_c) __attribute__((always_inline)) {
+    ot_zero<decltype(i_c)::value>();
+  });
+#pragma unroll
+  for (int ds = 0; ds < NDS; ++ds) {
+    asm volatile("" : "+a"(kf[ds]));
+    asm volatile("" : "+a"(vf[ds]));
+  }
+
+  // LDS offsets of the row reads and of the two transposed reads per fragment
+  int rro[NDS], tra[NDT], trb[NDT];
+  {
+    const int r = sigma32(ln);
+#pragma unroll
+    for (int ds = 0; ds < NDS; ++ds) rro[ds] = r * RB + (((2 * ds + lg) ^ swz<D>(r)) * 16);
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) {
+      tra[dt] = tr_offset<D>(lane, dt);
+      trb[dt] = tra[dt] ^ 16;
+    }
+  }
+  const float c2 = a.scale_log2;
+  const DA_LDS char* lds0 = (const DA_LDS char*)&smem[0][0][0];
+  const int sto = TB + wave * 256 + 32 * lg;
+
+  // Element e of a lane's score tile is row r0 + 16 (e / 8) + 8 lg + e % 8 of
+  // the unit, key `key`: masked to -inf outside the rows that see the key
+  // (boundary steps only; wave-uniform test)
+  auto mask = [&](int r0, f32x16& x) __attribute__((always_inline)) {
+    if (kw + 31 <= r0 && r0 + RT - 1 < rhi_w) return;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int row = r0 + 16 * (e >> 3) + 8 * lg + (e & 7);
+      x[e] = row >= key && row < rhi ? x[e] : -INFINITY;
+    }
+  };
+  // One unit: softmax, dV and dK of unit `u` (scores x, y), scores of unit
+  // u + 1 (whose slot holds zeros after the last unit: unused). With ISSUE the
+  // next two units of the stream are issued on the way, one operation a slot.
+  auto iter = [&](int u, auto issue_tag, f32x16& x, f32x16& y, f32x16& nx, f32x16& ny) __attribute__((always_inline)) {
+    constexpr bool ISSUE = decltype(issue_tag)::value;
+    const DA_LDS char* cur = lds0 + (u & (NSLOT - 1)) * (2 * TS);
+    const DA_LDS char* nxt = lds0 + ((u + 1) & (NSLOT - 1)) * (2 * TS);
+    const DA_LDS char* st = cur + sto;
+    auto rowfrag = [&](int q) __attribute__((always_inline)) -> u32x4 {
+      return *(const DA_LDS u32x4*)(nxt + rro[q / 2] + (q % 2) * TS);
+    };
+    // transposed fragment f: half f / 8, dims tile (f % 8) / 2, dO^T then Q^T
+    auto trfrag = [&](int f) __attribute__((always_inline)) -> u32x4 {
+      const int half = f / 8, dt = (f % 8) / 2;
+      const DA_LDS char* t = cur + (f % 2 == 0 ? TS : 0) + 16 * half * RB;
+      const u32x2 v0 = read_tr16(t + tra[dt]);
+      const u32x2 v1 = read_tr16(t + trb[dt] + 4 * RB);
+      return (u32x4){v0[0], v0[1], v1[0], v1[1]};
+    };
+    constexpr int AH = 4, NR = AH + 1;
+    // element e: FMA in slot xs - 1, exponential and y - D in slot xs, their
+    // product in slot xs + 1, the pair's packs in slot xs + 2 (half 0 by slot
+    // 13, half 1 by slot 21: two slots and more before their first MFMAs)
+    auto xs = [](int e) constexpr { return 5 + 15 * e / 16; };
+    u32x4 fr[NR], tr[NR];
+    f32x4 ls[4], dd[4];
+    float fv[16], pv[16], yd[16], sv[16];
+    uint32_t pf[8], sf[8];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      nx[j] = 0.f;
+      ny[j] = 0.f;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    StaticFor<0, 33>::run([&](auto i_c) __attribute__((always_inline)) {
+      constexpr int sl = decltype(i_c)::value - 1;
+      if constexpr (sl == -1) {
+#pragma unroll
+        for (int q = 0; q < AH; ++q) fr[q] = rowfrag(q);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          ls[j] = *(const DA_LDS f32x4*)(st + 64 * (j / 2) + 16 * (j % 2));
+          dd[j] = *(const DA_LDS f32x4*)(st + TS + 64 * (j / 2) + 16 * (j % 2));
+        }
+      }
+      if constexpr (ISSUE) {
+        if constexpr (sl == 0 || sl == 8) next_unit();
+        if constexpr (sl >= 1 && sl < 1 + UNIT_VM) issue_op(std::integral_constant<int, sl - 1>());
+        if constexpr (sl >= 9 && sl < 9 + UNIT_VM) issue_op(std::integral_constant<int, sl - 9>());
+      }
+      if constexpr (sl >= 0 && sl + AH < 16) fr[(sl + AH) % NR] = rowfrag(sl + AH);
+      if constexpr (sl >= 16 - AH && sl < 32 - AH) tr[(sl - 16 + AH) % NR] = trfrag(sl - 16 + AH);
+      if constexpr (sl >= 0 && sl < 16) {
+        if constexpr (sl % 2 == 0) nx = E::mfma(fr[sl % NR], kf[sl / 2], nx);
+        else ny = E::mfma(fr[sl % NR], vf[sl / 2], ny);
+      } else if constexpr (sl >= 16) {
+        constexpr int f = sl - 16, half = f / 8, dt = (f % 8) / 2;
+        if constexpr (f % 2 == 0)
+          ot_mfma<T, dt>(tr[f % NR], (u32x4){pf[4 * half], pf[4 * half + 1], pf[4 * half + 2], pf[4 * half + 3]});
+        else
+          ot_mfma<T, NDT + dt>(tr[f % NR], (u32x4){sf[4 * half], sf[4 * half + 1], sf[4 * half + 2], sf[4 * half + 3]});
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        if (xs(e) - 1 == sl) fv[e] = fmaf(x[e], c2, -ls[e / 4][e % 4]);
+        if (xs(e) == sl) {
+          pv[e] = fast_exp2(fv[e]);
+          yd[e] = y[e] - dd[e / 4][e % 4];
+        }
+        if (xs(e) + 1 == sl) sv[e] = pv[e] * yd[e];
+        if (e % 2 == 1 && xs(e) + 2 == sl) {
+          pf[e / 2] = E::pack2(pv[e - 1], pv[e]);
+          sf[e / 2] = E::pack2(sv[e - 1], sv[e]);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+
+  if (n > 0) {
+    wait_vm<3 * UNIT_VM>();       // units 0 - 2
+    lds_barrier();
+    f32x16 xa, ya, xb, yb;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      xa[j] = 0.f;
+      ya[j] = 0.f;
+    }
+#pragma unroll
+    for (int ds = 0; ds < NDS; ++ds) {
+      xa = E::mfma(*(const DA_LDS u32x4*)(lds0 + rro[ds]), kf[ds], xa);
+      ya = E::mfma(*(const DA_LDS u32x4*)(lds0 + rro[ds] + TS), vf[ds], ya);
+    }
+    mask(r_first, xa);
+    // row step of the unit whose scores come next
+    int m_g = 1, m_r0 = r_first;
+    auto step = [&]() __attribute__((always_inline)) -> int {
+      if (m_g == a.G) {
+        m_g = 0;
+        m_r0 = m_r0 + RT <= c_end ? m_r0 + RT : c_start;
+      }
+      ++m_g;
+      return m_r0;
+    };
+    for (int u = 0; u < n; u += 2) {
+      iter(u, std::true_type(), xa, ya, xb, yb);
+      mask(step(), xb);
+      if (u + 1 < n) {
+        iter(u + 1, std::false_type(), xb, yb, xa, ya);
+        mask(step(), xa);
+      }
+      // units u + 4 and u + 5 must have landed (u + 6 and u + 7 may still be in
+      // flight); slots u and u + 1 are free behind the barrier
+      wait_vm<2 * UNIT_VM>();
+      lds_barrier();
+    }
+  }
+  // no DMA may outlive the workgroup's LDS
+  wait_dma();
+
+  f32x16 adk[NDT], adv[NDT];
+  ot_pad();
+  StaticFor<0, NDT>::run([&](auto dt_c) __attribute__((always_inline)) {
+    constexpr int dt = decltype(dt_c)::value;
+    adv[dt] = ot_read<dt>();
+    adk[dt] = ot_read<NDT + dt>();
+  });
+  dkdv_store<T, D>(a, adk, adv, b, hk, bh, blk, item, key, wave * 32 + ln, lg);
 }
 
 // dK, dV of the keys of blocks cut into several items (every key, or the
@@ -1133,7 +1463,10 @@ void launch_bwd(const BwdArgs& a, hipStream_t s) {
                        dim3(RED), 0, s, a);
   }
   const int gk = a.B * a.Hkv * a.items_per_bh;
-  hipLaunchKernelGGL((dkdv_kernel<T, D, ROWS>), dim3((gk + 7) / 8 * 8), dim3(NTHR), 0, s, a);
+  if constexpr (D == 128 && !ROWS)
+    hipLaunchKernelGGL((dkdv_pipe_kernel<T>), dim3((gk + 7) / 8 * 8), dim3(NTHR), 0, s, a);
+  else
+    hipLaunchKernelGGL((dkdv_kernel<T, D, ROWS>), dim3((gk + 7) / 8 * 8), dim3(NTHR), 0, s, a);
   const int64_t tasks = (int64_t)a.B * a.Hkv * a.red_keys * (D / 8);
   if (tasks > 0)
     hipLaunchKernelGGL((dkdv_reduce_kernel<T, D>), dim3((unsigned)((tasks + RED - 1) / RED)),

@@ -134,6 +134,32 @@ __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, DA_LDS void* lds
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds, 16, voff, 0, 0, NT ? 2 : 0);
 }
 
+// The same DMAs outside the compiler's wait tracking, which otherwise puts a
+// wait for every DMA in flight before the next transposed LDS read: the caller
+// waits (vmcnt) and synchronises before the data is read. `r` holds the words
+// of a raw buffer resource, `lds` the LDS byte address (both wave-uniform);
+// there is no register result for the compiler to reuse early. M0 (reserved,
+// so not a clobber) is set in the same statement: a kernel uses either these
+// or the tracked DMAs, whose M0 the compiler keeps.
+__device__ __forceinline__ u32x4 rsrc_words(const void* base, uint32_t bytes) {
+  const uint64_t p = (uint64_t)base;
+  return (u32x4){(uint32_t)p, (uint32_t)(p >> 32) & 0xffffu, bytes, 0x00020000u};
+}
+__device__ __forceinline__ void dma16_untracked(u32x4 r, uint32_t lds, uint32_t voff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+               :: "s"(lds), "v"(voff), "s"(r) : "memory");
+}
+__device__ __forceinline__ void dma4_untracked(u32x4 r, uint32_t lds, uint32_t voff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
+               :: "s"(lds), "v"(voff), "s"(r) : "memory");
+}
+
+// Barrier of the workgroup that waits for this wave's LDS reads only: the
+// DMAs in flight stay in flight (__syncthreads would wait for them too).
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // Division by a divisor fixed for a launch (d >= 1) of dividends in
 // [0, 2^31), by multiply and shift: q = (mulhi(n, m) + n) >> s with
 // s = ceil(log2 d) and m = floor(2^32 (2^s - d) / d) + 1 (Granlund and

@@ -62,6 +62,14 @@ def test_rows(gpu, B, H, Hkv, S, D, dtype, rows):
     (1, 2, 2, 400, 128, torch.float16, 1000, 0),       # window past the sequence
     (2, 8, 2, 640, 32, torch.bfloat16, 128, 300),      # three sink blocks
     (1, 4, 4, 96, 64, torch.bfloat16, 64, 8),          # one key block
+    # head_dim 128 (the unit ring of dkdv_pipe_kernel): five heads and a last
+    # step of 8 rows, eight heads, one head with fewer units than ring slots,
+    # a window shorter than its block, sinks ending inside a wave's keys
+    (1, 5, 1, 1000, 128, torch.bfloat16, 300, 70),
+    (2, 8, 1, 500, 128, torch.float16, 128, 0),
+    (1, 3, 3, 70, 128, torch.bfloat16, 64, 0),
+    (1, 2, 1, 333, 128, torch.bfloat16, 40, 45),
+    (1, 4, 2, 2100, 128, torch.bfloat16, 256, 128),
 ])
 def test_key_sparse(gpu, B, H, Hkv, S, D, dtype, window, sink):
     from delta_attention import ops
