@@ -23,7 +23,7 @@
 //     LDS reads. It also writes rowsum(dO * O) for the other kernel. Long
 //     key lists (selected rows) are split; the splits' fp32 partial dQ are
 //     summed by dq_reduce_kernel.
-//   * dkdv_kernel: one workgroup per 128 keys (32 per wave, K and V fragments
+//   * dkdv_kernel (head_dim 32 and 64): one workgroup per 128 keys (32 per wave, K and V fragments
 //     in registers) and a chunk of the rows that see them; per 32-row tile and
 //     query head it stages Q, dO, lse and rowsum(dO * O) in LDS (by
 //     buffer-load DMA into two stages, the next tile's rows in flight under
@@ -32,8 +32,8 @@
 //     dK^T += Q^T dS from transposed LDS reads. Sink keys are seen by every
 //     later row, so their row range is cut into chunks like any other; each
 //     chunk writes fp32 partials that dkdv_reduce_kernel sums per key.
-//   * dkdv_pipe_kernel: the same for key-sparse attention at head_dim 128, as
-//     one static schedule over a ring of (row step, head) units.
+//   * dkdv_pipe_kernel: the same at head_dim 128, as one static schedule over a
+//     ring of (row step, head) units (selected rows from a gathered copy of q).
 // Every MFMA is v_mfma_f32_32x32x16 (bf16 or fp16 operands, fp32 accumulate).
 #include <algorithm>
 #include <atomic>
@@ -87,6 +87,7 @@ struct BwdArgs {
   const int64_t* row_last;       // selected rows: last visible key, ascending
   int accumulate;                // outputs: out = rnd(out + rnd(grad))
   int q32;                       // selected rows: every q row of a head within 32-bit byte offsets
+  void* q_gather;                // selected rows at head_dim 128: their q rows [B, Hq, n_rows, D]
   // dq kernel
   int n_mtiles, n_splits, chunk;
   float* dq_part;                // [item][BM][D] when n_splits > 1
@@ -899,8 +900,7 @@ __global__ __launch_bounds__(NTHR, 1) void dkdv_kernel(BwdArgs a) {
   dkdv_store<T, D>(a, adk, adv, b, hk, bh, blk, item, key, wave * 32 + ln, lg);
 }
 
-// dkdv_kernel for the key-sparse attention at head_dim 128, as one static
-// schedule. With one wave per SIMD nothing hides a fragment read or the
+// dkdv_kernel for head_dim 128, as one static schedule. With one wave per SIMD nothing hides a fragment read or the
 // softmax chain: the compiler's order of dkdv_kernel waits for LDS 36 times
 // per head and took about 2900 cycles for its 32 MFMAs (1024 cycles). Here
 //  * the (32-row step, query head) pairs of the item, heads innermost, are one
@@ -916,14 +916,19 @@ __global__ __launch_bounds__(NTHR, 1) void dkdv_kernel(BwdArgs a) {
 //    the K and V fragments in the AGPRs below them.
 // Rows past the chunk end read as zero and are masked like rows out of a key's
 // window.
-// 32 heads / 8 at 32768 rows, window 2048: both key-sparse backward kernels
+// 638 selected rows of 32 heads at 32768 keys: backward of the rows 972 -> 899
+// us, 8 / 8 heads at 16384 199 -> 165 us (the old kernel gathered q rows by
+// DMA). 32 heads / 8 at 32768 rows, window 2048: both key-sparse backward kernels
 // 4.59 -> 4.16 ms (this one about 2.73 -> 2.3); 8 / 8 heads at 16384 rows 858
 // -> 580 us. On copies that drop work: no DMA -350 us, no transposed reads
 // -190, no exponentials -150; what is left, 1.7 ms, is the MFMA issue rate of
 // one wave per SIMD (about 50 cycles each). Issued between the iterations
 // instead of one a slot, the DMAs cost 160 us; plain row order instead of the
 // cyclic one 65 us.
-template <typename T>
+// ROWS: selected rows, list positions in place of rows: q comes from the
+// gathered copy (as contiguous as dO), and since the limits ascend, a key is
+// seen by the positions from the first whose limit reaches it on.
+template <typename T, bool ROWS>
 __global__ __launch_bounds__(NTHR, 1) void dkdv_pipe_kernel(BwdArgs a) {
   using E = Elt<T>;
   constexpr int D = 128, NDS = D / 16, NDT = D / 32, DCH = D / 8, RB = 2 * D;
@@ -965,13 +970,34 @@ __global__ __launch_bounds__(NTHR, 1) void dkdv_pipe_kernel(BwdArgs a) {
     const int tq = kk + a.window - a.q_block;
     return tq < 0 ? 0 : (tq / a.q_block + 1) * a.q_block;
   };
-  const int p_end = k0 < a.sink ? a.n_rows - 1
-                                : min(a.n_rows, row_hi(min(k0 + KT - 1, a.n_kv - 1))) - 1;
-  const int c_start = k0 + c * a.rpc;
+  // first position in [p, e) whose limit reaches kk
+  auto first_of = [&](int kk, int p, int e) -> int {
+    while (p < e) {
+      const int mid = (p + e) >> 1;
+      const int64_t lim = min(a.row_last[mid], (int64_t)(a.n_kv - 1));
+      if (lim >= kk) e = mid;
+      else p = mid + 1;
+    }
+    return p;
+  };
+  const int p_start = ROWS ? first_of(k0, 0, a.n_rows) : k0;
+  const int p_end = ROWS || k0 < a.sink ? a.n_rows - 1
+                                        : min(a.n_rows, row_hi(min(k0 + KT - 1, a.n_kv - 1))) - 1;
+  const int c_start = p_start + c * a.rpc;
   const int c_end = min(p_end, c_start + a.rpc - 1);
-  const int rhi = min(c_end + 1, key < a.sink ? 0x7fffffff : row_hi(key));
-  // rows below see every key of the wave that is not above them
-  const int rhi_w = min(c_end + 1, kw + 31 < a.sink ? 0x7fffffff : row_hi(kw));
+  // key `key` is seen by the rows rlo .. rhi - 1, every key of the wave by the
+  // rows rlo_w .. rhi_w - 1. Distinct limits put a block's keys within the KT
+  // positions from p_start on; repeated ones may reach further.
+  int rlo = key, rlo_w = kw + 31, rhi = c_end + 1, rhi_w = c_end + 1;
+  if constexpr (ROWS) {
+    int e = a.n_rows;
+    if (p_start + KT < a.n_rows && a.row_last[p_start + KT] >= k0 + KT - 1) e = p_start + KT;
+    rlo = first_of(key, p_start, e);
+    rlo_w = __builtin_amdgcn_readlane(rlo, 31);
+  } else {
+    rhi = min(rhi, key < a.sink ? 0x7fffffff : row_hi(key));
+    rhi_w = min(rhi_w, kw + 31 < a.sink ? 0x7fffffff : row_hi(kw));
+  }
   const int n_steps = c_end >= c_start ? (c_end - c_start) / RT + 1 : 0;
   const int n = n_steps * a.G;
   // The row steps are walked cyclically from the one whose number (row / 32)
@@ -979,12 +1005,17 @@ __global__ __launch_bounds__(NTHR, 1) void dkdv_pipe_kernel(BwdArgs a) {
   // each other on an XCD, each starting 128 rows after the last, then read the
   // same rows at the same time, and the rows come from L2 (in plain order the
   // 32 blocks of an XCD read 12 MB of rows apart).
-  const int r_first = n_steps > 0 ? c_start + (n_steps - 1 - (c_start / RT + n_steps - 1) % n_steps) * RT : 0;
+  // (selected rows keep their order: neighbouring blocks start at the same ones)
+  const int r_first = ROWS || n_steps == 0
+                          ? c_start
+                          : c_start + (n_steps - 1 - (c_start / RT + n_steps - 1) % n_steps) * RT;
 
   // ---- unit stream: DMA of unit u (row step, head) into slot u % 8, issued
   //      in order ----
-  const uint32_t qrow_b = (uint32_t)(a.qs_s * (int64_t)esz), grow_b = (uint32_t)(a.gs_s * (int64_t)esz);
-  const char* qb0 = (const char*)a.q + ((int64_t)b * a.qs_b + (int64_t)hk * a.G * a.qs_h) * esz;
+  const int64_t qs_s = ROWS ? D : a.qs_s, qs_h = ROWS ? (int64_t)a.n_rows * D : a.qs_h;
+  const int64_t qs_b = ROWS ? a.Hq * qs_h : a.qs_b;
+  const uint32_t qrow_b = (uint32_t)(qs_s * (int64_t)esz), grow_b = (uint32_t)(a.gs_s * (int64_t)esz);
+  const char* qb0 = (const char*)(ROWS ? a.q_gather : a.q) + ((int64_t)b * qs_b + (int64_t)hk * a.G * qs_h) * esz;
   const char* gb0 = (const char*)a.dout + ((int64_t)b * a.gs_b + (int64_t)hk * a.G * a.gs_h) * esz;
   const int64_t st0 = ((int64_t)b * a.Hq + (int64_t)hk * a.G) * a.n_rows;
   uint32_t qoff[NDMA], goff[NDMA];
@@ -997,7 +1028,7 @@ __global__ __launch_bounds__(NTHR, 1) void dkdv_pipe_kernel(BwdArgs a) {
   }
   const uint32_t soff = lane < RT ? (uint32_t)lane * 4 : 0xfffffff0u;
   int u_next = 0, u_g = 0, u_r0 = r_first;
-  const char* u_q = qb0 + (int64_t)r_first * a.qs_s * esz;
+  const char* u_q = qb0 + (int64_t)r_first * qs_s * esz;
   const char* u_d = gb0 + (int64_t)r_first * a.gs_s * esz;
   int64_t u_s = st0 + r_first;
   u32x4 rq, rg, rl, rd;
@@ -1012,13 +1043,13 @@ __global__ __launch_bounds__(NTHR, 1) void dkdv_pipe_kernel(BwdArgs a) {
     rd = rsrc_words(a.dvec + u_s, nrow * 4);
     u_lds = lds_w + (uint32_t)(u_next & (NSLOT - 1)) * (2 * TS);
     ++u_next;
-    u_q += a.qs_h * (int64_t)esz;
+    u_q += qs_h * (int64_t)esz;
     u_d += a.gs_h * (int64_t)esz;
     u_s += a.n_rows;
     if (++u_g == a.G) {
       u_g = 0;
       u_r0 = u_r0 + RT <= c_end ? u_r0 + RT : c_start;
-      u_q = qb0 + (int64_t)u_r0 * a.qs_s * esz;
+      u_q = qb0 + (int64_t)u_r0 * qs_s * esz;
       u_d = gb0 + (int64_t)u_r0 * a.gs_s * esz;
       u_s = st0 + u_r0;
     }
@@ -1078,11 +1109,11 @@ __global__ __launch_bounds__(NTHR, 1) void dkdv_pipe_kernel(BwdArgs a) {
   // the unit, key `key`: masked to -inf outside the rows that see the key
   // (boundary steps only; wave-uniform test)
   auto mask = [&](int r0, f32x16& x) __attribute__((always_inline)) {
-    if (kw + 31 <= r0 && r0 + RT - 1 < rhi_w) return;
+    if (rlo_w <= r0 && r0 + RT - 1 < rhi_w) return;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       const int row = r0 + 16 * (e >> 3) + 8 * lg + (e & 7);
-      x[e] = row >= key && row < rhi ? x[e] : -INFINITY;
+      x[e] = row >= rlo && row < rhi ? x[e] : -INFINITY;
     }
   };
   // One unit: softmax, dV and dK of unit `u` (scores x, y), scores of unit
@@ -1213,6 +1244,21 @@ __global__ __launch_bounds__(NTHR, 1) void dkdv_pipe_kernel(BwdArgs a) {
     adk[dt] = ot_read<NDT + dt>();
   });
   dkdv_store<T, D>(a, adk, adv, b, hk, bh, blk, item, key, wave * 32 + ln, lg);
+}
+
+// The selected rows' q rows as [B, Hq, n_rows, D], 8 dims per thread.
+template <int D>
+__global__ __launch_bounds__(RED) void gather_q_kernel(BwdArgs a) {
+  constexpr int CPR = D / 8;
+  const int64_t task = (int64_t)blockIdx.x * RED + threadIdx.x;
+  if (task >= (int64_t)a.B * a.Hq * a.n_rows * CPR) return;
+  const int c = (int)(task % CPR);
+  const int64_t row = task / CPR;
+  const int i = (int)(row % a.n_rows);
+  const int h = (int)(row / a.n_rows % a.Hq), b = (int)(row / a.n_rows / a.Hq);
+  const int64_t qrow = min(max(a.q_rows[i], (int64_t)0), (int64_t)(a.n_q - 1));
+  ((u32x4*)a.q_gather)[task] = *(const u32x4*)((const char*)a.q +
+      ((int64_t)b * a.qs_b + (int64_t)h * a.qs_h + qrow * a.qs_s + 8 * c) * 2);
 }
 
 // dK, dV of the keys of blocks cut into several items (every key, or the
@@ -1448,8 +1494,7 @@ size_t bwd_ws_bytes(int B, int Hq, int Hkv, int n_rows, int n_kv, int D, const D
     bytes += (size_t)B * Hkv * dq.n_splits * dq.n_mtiles * BM * D * sizeof(float);
   bytes = (bytes + 255) / 256 * 256;
   bytes += (size_t)B * Hkv * kv.part_per_bh * 2 * KT * D * sizeof(float);
-  (void)rows;
-  (void)esz;
+  if (rows && D == 128) bytes += (size_t)B * Hq * n_rows * D * esz;   // gathered q rows
   return bytes;
 }
 
@@ -1463,9 +1508,13 @@ void launch_bwd(const BwdArgs& a, hipStream_t s) {
                        dim3(RED), 0, s, a);
   }
   const int gk = a.B * a.Hkv * a.items_per_bh;
-  if constexpr (D == 128 && !ROWS)
-    hipLaunchKernelGGL((dkdv_pipe_kernel<T>), dim3((gk + 7) / 8 * 8), dim3(NTHR), 0, s, a);
-  else
+  if constexpr (D == 128) {
+    if constexpr (ROWS) {
+      const int64_t pieces = (int64_t)a.B * a.Hq * a.n_rows * (D / 8);
+      hipLaunchKernelGGL((gather_q_kernel<D>), dim3((unsigned)((pieces + RED - 1) / RED)), dim3(RED), 0, s, a);
+    }
+    hipLaunchKernelGGL((dkdv_pipe_kernel<T, ROWS>), dim3((gk + 7) / 8 * 8), dim3(NTHR), 0, s, a);
+  } else
     hipLaunchKernelGGL((dkdv_kernel<T, D, ROWS>), dim3((gk + 7) / 8 * 8), dim3(NTHR), 0, s, a);
   const int64_t tasks = (int64_t)a.B * a.Hkv * a.red_keys * (D / 8);
   if (tasks > 0)
@@ -1577,7 +1626,8 @@ static void place_workspace(BwdArgs& a, const DqPlan& dq, const KvPlan& kv, int 
   if (dq.n_splits > 1) off += (size_t)a.B * a.Hkv * dq.n_splits * dq.n_mtiles * BM * D * sizeof(float);
   off = (off + 255) / 256 * 256;
   a.kv_part = (float*)(p + off);
-  (void)rows;
+  off += (size_t)a.B * a.Hkv * kv.part_per_bh * 2 * KT * D * sizeof(float);
+  a.q_gather = rows && D == 128 ? p + off : nullptr;
 }
 
 extern "C" int da_sparse_attn_bwd(const void* q, const void* k, const void* v, const void* o,

@@ -44,6 +44,10 @@ def _inputs(B, H, Hkv, S, D, dtype, n):
     (1, 4, 2, 64, 32, torch.bfloat16, list(range(64))),          # one tile
     (1, 5, 1, 900, 128, torch.bfloat16, [0, 1, 63, 64, 255, 256, 257, 899]),
     (1, 8, 8, 1300, 64, torch.bfloat16, list(range(0, 1300, 3))),
+    (1, 5, 1, 1300, 128, torch.bfloat16, list(range(300, 1300, 3))),     # first keys seen by every row
+    (2, 8, 1, 700, 128, torch.float16, list(range(0, 700, 64)) + list(range(690, 700))),
+    (1, 2, 2, 300, 128, torch.bfloat16, list(range(300))),               # every row
+    (1, 3, 3, 500, 128, torch.bfloat16, [499]),
 ])
 def test_rows(gpu, B, H, Hkv, S, D, dtype, rows):
     from delta_attention import ops
