@@ -11,11 +11,14 @@
 // Each chunk's stride depends on the previous chunk's dense rows, so
 // computing them chunk by chunk makes a chain of small kernel (2) launches
 // (at 128K, 32 launches that together take half again as long as one launch
-// over the same rows). When gamma0 divides adapt_chunk, the dense rows at
-// every multiple of gamma0 below s_p are computed ahead in one launch; a
-// chunk whose stride is a multiple of gamma0 (the starting stride and every
-// doubling of it) takes its anchors' rows from there, any other chunk
-// recomputes its anchors. Per chunk c:
+// over the same rows). When gamma0 divides adapt_chunk, the dense rows at every
+// multiple of gamma0 below s_p are computed ahead in one launch; a chunk whose
+// stride is a multiple of gamma0 (the starting stride and every doubling of it)
+// takes its anchors' rows from there, any other chunk recomputes its anchors.
+// The launch follows the first of the early chunks whose decision leaves the
+// next chunk such a stride (before chunk 0 in short layers): where the stride
+// falls at once and stays low the rows ahead would be wasted, 0.23 of 2.9 ms at
+// 40K tokens (2.95 -> 2.72 ms without them). Per chunk c:
 //   kernel (2) over the chunk's anchors when it recomputes them (a launch
 //     over a device-held row count that is zero otherwise), into one of two
 //     row buffers;
@@ -48,6 +51,11 @@ int delta_add_chunk(void* out, const int64_t o_str[3], const void* dense,
 
 namespace {
 
+// The rows ahead wait for a chunk to show that they will be used in layers of
+// at least AHEAD_LAZY_CHUNKS chunks (two chunks at 6001 tokens: 313 us with the
+// rows ahead first, 323 us waiting), behind one of the first AHEAD_TRIES
+// chunks' decisions (a launch over no rows costs each of them a few us).
+constexpr int AHEAD_LAZY_CHUNKS = 4, AHEAD_TRIES = 4;
 constexpr int NEV = 4;      // events per ring; a ring slot is reused NEV chunks later
 
 // Rows per key-sparse launch on the second stream, in whole chunks of at least
@@ -92,7 +100,7 @@ AdaptPlan plan_adapt(int B, int Hq, int Hkv, int S, int D, int s_p, int adapt_ch
   p.off_rows = o;  o = up256(o + (size_t)std::max(p.nc, 1) * p.max_n * 8);
   p.off_tail = o;  o = up256(o + (size_t)p.cut_n * 8);
   p.off_ahead_rows = o; o = up256(o + (size_t)p.n_ahead * 8);
-  p.off_state = o; o = up256(o + 5 * sizeof(int));
+  p.off_state = o; o = up256(o + 7 * sizeof(int));
   p.off_sel = o;   o = up256(o + (size_t)2 * std::max(p.nc, 1) * sizeof(int));
   p.off_cos = o;   o = up256(o + (size_t)B * std::max(p.max_n - 1, 1) * Hq * sizeof(float));
   p.dense_bytes = up256((size_t)B * Hq * p.max_n * D * esz);
@@ -122,18 +130,22 @@ AdaptPlan plan_adapt(int B, int Hq, int Hkv, int S, int D, int s_p, int adapt_ch
 __global__ __launch_bounds__(256) void adapt_init_kernel(int64_t* rows0, int max_n, int n0,
                                                          int gamma0, int64_t* tail, int s_p,
                                                          int cut_n, int64_t* ahead, int n_ahead,
-                                                         int* state) {
+                                                         int lazy, int* state) {
   for (int j = threadIdx.x; j < max_n; j += 256)
     rows0[j] = j < n0 ? (int64_t)j * gamma0 : (int64_t)-1;
   for (int j = threadIdx.x; j < cut_n; j += 256) tail[j] = (int64_t)s_p + j;
   for (int j = threadIdx.x; j < n_ahead; j += 256) ahead[j] = (int64_t)j * gamma0;
   if (threadIdx.x == 0) {
-    // {stride, anchors, anchors to recompute, first slot ahead (-1: none), slot step}
+    // {stride, anchors, anchors to recompute, first slot ahead (-1: none), slot
+    // step, have rows ahead, rows ahead to compute}
+    const bool have = n_ahead > 0 && !lazy;
     state[0] = gamma0;
     state[1] = n0;
-    state[2] = n_ahead > 0 ? 0 : n0;
-    state[3] = n_ahead > 0 ? 0 : -1;
+    state[2] = have ? 0 : n0;
+    state[3] = have ? 0 : -1;
     state[4] = 1;
+    state[5] = have;
+    state[6] = 0;
   }
 }
 
@@ -184,7 +196,7 @@ extern "C" int da_adapt_layer_fwd(const void* q, const void* k, const void* v, v
   void* ws_ahead = ws + p.off_ws_ahead;
   void* ws_tail = ws + p.off_ws_tail;
   const int max_n = p.max_n;
-  const bool use_ahead = p.n_ahead > 0;
+  const bool use_ahead = p.n_ahead > 0, lazy = use_ahead && p.nc >= AHEAD_LAZY_CHUNKS;
   // strides (batch, head, row) for kernel (2) and the broadcast, (batch, row,
   // head) for the cosines
   const int64_t dn_bhr[3] = {(int64_t)Hq * max_n * D, (int64_t)max_n * D, D};
@@ -215,13 +227,13 @@ extern "C" int da_adapt_layer_fwd(const void* q, const void* k, const void* v, v
   const int n0 = p.nc > 0 ? std::min((std::min(adapt_chunk, s_p) + gamma0 - 1) / gamma0, max_n) : 0;
   (void)hipGetLastError();
   hipLaunchKernelGGL(adapt_init_kernel, dim3(1), dim3(256), 0, st, rows_all, max_n, n0, gamma0,
-                     tail, s_p, p.cut_n, ahead_rows, p.n_ahead, state);
+                     tail, s_p, p.cut_n, ahead_rows, p.n_ahead, lazy ? 1 : 0, state);
   if (hipGetLastError() != hipSuccess) rc = DA_ERR_LAUNCH;
   // the second stream starts once the inputs and the first chunk's state are ready
   if (rc == DA_OK && side &&
       !(ok(hipEventRecord(ev_join, st)) && ok(hipStreamWaitEvent(side, ev_join, 0))))
     rc = DA_ERR_LAUNCH;
-  if (rc == DA_OK && use_ahead)
+  if (rc == DA_OK && use_ahead && !lazy)
     rc = da_qsparse_attn_fwd(q, k, v, ahead_rows, ahead_rows, 0, p.n_ahead, B, Hq, Hkv, S, s_p, D,
                              q_str, k_str, v_str, ahead, ah_bhr, DA_EPI_OUTPUT, 0, nullptr,
                              nullptr, sm_scale, ws_ahead, p.ws_ahead_bytes, dtype, st);
@@ -244,6 +256,8 @@ extern "C" int da_adapt_layer_fwd(const void* q, const void* k, const void* v, v
   ad.log_mean = log_mean; ad.log_min = log_min; ad.log_gamma = log_gamma; ad.log_n = log_n;
   ad.full_state = true;
   ad.spec_gamma = use_ahead ? gamma0 : 0;
+  ad.n_ahead = p.n_ahead;
+  ad.try_chunks = lazy ? AHEAD_TRIES : 0;
   ad.sel_log = use_ahead ? sel_log : nullptr;
 
   // chunk c's recompute launch and its decision chain (the key-sparse rows
@@ -278,11 +292,17 @@ extern "C" int da_adapt_layer_fwd(const void* q, const void* k, const void* v, v
     // launches' time beside the key-sparse launches did not change)
     if ((r = adapt_step_launch(cs, ad, p.n_live, dtype, st)) != DA_OK) return r;
     if (side && !ok(hipEventRecord(ev_next[c % NEV], st))) return DA_ERR_LAUNCH;
-    return use_ahead
+    r = use_ahead
         ? delta_add_chunk(out, o_str, ahead, ah_bhr, sel_log + 2 * c, dense, dn_bhr, rows_c,
                           log_n + c, max_n, end, s_p, B, Hq, D, p.n_live, dtype, st)
         : delta_add_chunk(out, o_str, dense, dn_bhr, nullptr, nullptr, nullptr, rows_c,
                           log_n + c, max_n, end, s_p, B, Hq, D, p.n_live, dtype, st);
+    // the rows ahead, if this chunk's decision turned them on
+    if (r == DA_OK && lazy && c < AHEAD_TRIES && c + 1 < p.nc)
+      r = da_qsparse_attn_fwd_live(q, k, v, ahead_rows, ahead_rows, 0, p.n_ahead, p.n_ahead,
+                                   state + 6, B, Hq, Hkv, S, s_p, D, q_str, k_str, v_str, ahead,
+                                   ah_bhr, sm_scale, ws_ahead, p.ws_ahead_bytes, dtype, st);
+    return r;
   };
   const int per_launch =
       (int)std::max<int64_t>(1, ((int64_t)DA_ADAPT_SPARSE_ROWS + adapt_chunk - 1) / adapt_chunk);

@@ -150,8 +150,8 @@ struct AttnArgs {
   // [0, n_rows]) are computed; the items of their row tiles are spread over
   // the XCDs in contiguous ranges and the other blocks exit at once
   const int* n_rows_dev;
-  // live launches: the split length of a plan for n_live rows grows with the
-  // live row tiles (live_chunk): bound of a list's tiles, resident workgroups
+  // live launches planned for fewer rows: the split length grows with the live
+  // row tiles (live_chunk): bound of a list's tiles, resident workgroups (else 0)
   int vis, slots;
   // [item][ws_rows][D]: each row's O / l, float when part_f32, else elements
   void* part_o;
@@ -229,6 +229,7 @@ __device__ __forceinline__ void tile_list(int hi_max, int lo_min, int sink, int&
 // 64 rows, 256 rows x 32 heads at 40K keys took four rounds and 32 partials a
 // row.
 __device__ __forceinline__ int live_chunk(int chunk, int tiles, int vis, int slots) {
+  if (slots == 0) return chunk;   // planned for all the rows
   const int per_tile = max(slots / max(tiles, 1), 1);
   return max(chunk, min((vis + per_tile - 1) / per_tile, 80));
 }
@@ -1381,6 +1382,7 @@ struct QsparsePlan {
   size_t ws_bytes;
   int64_t vis;      // bound of a row tile's list
   bool f32;         // float partials
+  bool grow;        // live launches: split length from the live row tiles
 };
 
 // Rows per workgroup of a launch: for the head_dim-128 key-sparse launches
@@ -1410,6 +1412,7 @@ static QsparsePlan plan_qsparse(int B, int Hq, int Hkv, int n, int64_t vis, int 
                                 int min_chunk, int bm, int max_chunk = 0x7fffffff, bool f32 = false) {
   QsparsePlan p;
   p.f32 = f32;
+  p.grow = false;
   const int G = Hq / Hkv;
   p.bm = bm;
   p.n_mtiles = (int)(((int64_t)n * G + bm - 1) / bm);
@@ -1495,6 +1498,7 @@ static QsparsePlan plan_rows_live(int B, int Hq, int Hkv, int n, int n_live, int
                                   bool ends_seq) {
   if (n_live >= n || n_live < 1) return plan_rows(B, Hq, Hkv, n, Skv, D, ends_seq);
   QsparsePlan p = plan_rows(B, Hq, Hkv, n_live, Skv, D, false);
+  p.grow = true;
   const int G = Hq / Hkv;
   p.n_mtiles = (int)(((int64_t)n * G + p.bm - 1) / p.bm);
   const int64_t base = (int64_t)B * Hkv * p.n_mtiles;
@@ -1798,7 +1802,7 @@ static int run_qsparse(const QsparsePlan& p, const void* q, const void* k, const
   a.chunk = p.chunk; a.n_splits = p.n_splits; a.n_kv_dev = n_kv_dev;
   a.n_rows_dev = n_rows_dev;
   a.window = window; a.sink = sink;
-  a.vis = (int)p.vis; a.slots = (int)resident_slots(D);
+  a.vis = (int)p.vis; a.slots = p.grow ? (int)resident_slots(D) : 0;
   a.part_o = workspace; a.part_f32 = p.f32;
   a.ref_first = p.f32 && row_last;
   a.part_ml = (float*)((char*)workspace +
