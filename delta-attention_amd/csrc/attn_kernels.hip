@@ -72,10 +72,9 @@ namespace da {
 #ifndef DA_ROWS_MAX_TILES
 #define DA_ROWS_MAX_TILES 512
 #endif
-// Split items a decode-row launch aims for: one workgroup per resident slot
-// of the 256-CU gfx950 (two per CU), so the items run in a single round
-// (dense row over 131072 keys: 106-111 us against 118 us at 1024 items and
-// 131 us at 2048).
+// Split items of the decode plan that the static scratch is sized by
+// (plan_decode_short): one workgroup per resident slot of the 256-CU gfx950
+// (two per CU).
 #ifndef DA_DECODE_ITEMS
 #define DA_DECODE_ITEMS 512
 #endif

@@ -31,7 +31,7 @@ def kernels(tmp_path_factory):
     for m in re.finditer(r"^(_ZN2da15attn_fwd_kernel\S+):(.*?)^\.Lfunc_end", s, re.S | re.M):
         if "Li256E" in m.group(1):
             ks[m.group(1)] = m.group(2).splitlines()
-    assert len(ks) == 6, "three modes in bf16 and fp16"
+    assert len(ks) == 8, "four modes in bf16 and fp16"
     return ks
 
 
