@@ -803,13 +803,20 @@ def selected_rows(s: int, gamma: int, device: str) -> torch.Tensor:
 
 @functools.lru_cache(maxsize=64)
 def _selected_rows_of_stream(s: int, gamma: int, device: str, stream: int) -> torch.Tensor:
-    return selected_rows.__wrapped__(s, gamma, device)
+    # (a tensor made under inference_mode could not be saved for a later
+    # training step's backward)
+    with torch.inference_mode(False):
+        return selected_rows.__wrapped__(s, gamma, device)
 
 
 def selected_rows_here(s: int, gamma: int, device: torch.device) -> torch.Tensor:
     """selected_rows in a tensor of torch's current stream, kept per size and
     stream: a caller's every use of it is then ordered with its memory's reuse
-    (building it takes a blocking host-to-device copy, about 25 us)."""
+    (building it takes a blocking host-to-device copy, about 25 us). A graph
+    capture gets none of the kept lists: the graph would read its list after
+    the cache has dropped it. The copy of a new one is refused there."""
+    if torch.cuda.is_current_stream_capturing():
+        return selected_rows.__wrapped__(s, gamma, str(device))
     return _selected_rows_of_stream(s, gamma, str(device), _stream(device))
 
 

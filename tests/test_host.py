@@ -217,3 +217,29 @@ def test_fused_projection_params_keep_gradients():
     x = torch.randn(2, 16)
     sum(m(x).sum() for m in mods).backward()
     assert all(m.weight.grad is not None for m in mods)
+
+
+def test_kept_row_lists_serve_training_after_inference():
+    """A list first made under inference_mode is an ordinary tensor: a later
+    training step saves it for its backward."""
+    ops._selected_rows_of_stream.cache_clear()
+    with torch.inference_mode():
+        rows = ops._selected_rows_of_stream(300, 16, "cpu", 0)
+    assert not rows.is_inference()
+    assert rows is ops._selected_rows_of_stream(300, 16, "cpu", 0)
+    assert torch.equal(rows, ops.selected_rows.__wrapped__(300, 16, "cpu"))
+    ops._selected_rows_of_stream.cache_clear()
+
+
+def test_kept_row_lists_stay_out_of_graph_captures(monkeypatch):
+    """A captured graph never holds a list that the cache may drop."""
+    ops._selected_rows_of_stream.cache_clear()
+    monkeypatch.setattr(ops, "_stream", lambda dev: 0)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    dev = torch.device("cpu")
+    kept = ops.selected_rows_here(300, 16, dev)
+    assert kept is ops.selected_rows_here(300, 16, dev)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    captured = ops.selected_rows_here(300, 16, dev)
+    assert captured is not kept and captured.data_ptr() != kept.data_ptr()
+    ops._selected_rows_of_stream.cache_clear()
