@@ -102,12 +102,20 @@ constexpr float NEG_BIG = -1.0e30f;  // finite "minus infinity" for the running 
 // without row maxima that a max would have moved (P <= l). The probabilities
 // are packed into the element type for the PV product: fp16 holds at most
 // 65504, so its bound is 15.
+// A split that starts from the row max of the list's first tile (ref_first)
+// takes its own first max instead where that is more than `drop` below: fp16
+// probabilities under 2^-14 lose bits (64 rows against 12000 keys, key 0 13
+// nats above the others with a zero value: relative error 2.7e-3 from the
+// list's max, 6.6e-4 from the split's own). bf16 keeps its 8 bits down to
+// 2^-126.
 template <typename T> struct Rescale;
 template <> struct Rescale<__bf16> {
+  static constexpr float drop = INFINITY;
   static constexpr float thresh = 40.0f;
   static constexpr float lsum = 1099511627776.0f;   // 2^40
 };
 template <> struct Rescale<_Float16> {
+  static constexpr float drop = 4.0f;
   static constexpr float thresh = 15.0f;
   static constexpr float lsum = 32768.0f;           // 2^15
 };
@@ -879,8 +887,9 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
       // has the same exponent offset, hence the same rounding, as in the
       // key-sparse pass over those rows, whose rounding errors the delta
       // composition subtracts (with a max per split the composed output of a
-      // 1531-token layer was 6 % further from 64-bit arithmetic). One more
-      // score product per item, no extra wait.
+      // 1531-token layer was 6 % further from 64-bit arithmetic), unless its
+      // own keys lie far below (Rescale::drop). One more score product per
+      // item, no extra wait.
       const bool ref = !KSPARSE && a.ref_first && t_off > 0;
       if (ref) issue_ref(-t_off);
       wait_vmcnt<0>();
@@ -895,6 +904,16 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
       }
       qk(0, sa);
       mask(0, sa);
+      if constexpr (Rescale<T>::drop < INFINITY) {
+        if (ref) {
+#pragma unroll
+          for (int rg = 0; rg < RG; ++rg) {
+            // (O and l are still 0; a row without keys here keeps the list's)
+            const float mx = rowmax(sa[rg]);
+            m_i[rg] = mx > NEG_BIG && mx < m_i[rg] - Rescale<T>::drop ? mx : m_i[rg];
+          }
+        }
+      }
       update(sa);
       if (!EXACT) track = pending(1);
       __syncthreads();   // every wave is done with K stage 0 before it is refilled

@@ -3,6 +3,7 @@ lists cut into the shortest items, a plan of exactly one item per resident
 workgroup, one item per row tile, and the longest items of rows that end the
 sequence; against the oracle (tolerance: the layer's parity bar)."""
 
+import numpy as np
 import pytest
 import torch
 
@@ -39,3 +40,34 @@ def test_plan_edges(gpu, B, H, Hkv, n, N, D, selected):
         ref = O.qsparse_attention(np64(q[b:b + 1]), np64(k[b:b + 1]), np64(v[b:b + 1]),
                                   rows.cpu().numpy(), D ** -0.5)
         assert_close(np64(out[b:b + 1]), ref, what=f"B{B} n{n} N{N} D{D} batch {b}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("gap", [10.0, 13.0])
+def test_dominant_first_key(gpu, dtype, gap):
+    """Key 0 stands `gap` nats above the mean score of every other key (whose
+    scores are N(0, 1)) and has a zero value, so the output is the other keys'
+    probabilities alone. In fp16 only the split that holds key 0 may pack them
+    as subnormals (spacing 2^-24): with the 4-tile items of this plan 256 of
+    12000 keys, each off by 2^-24 / sqrt(12) rms, against probabilities of
+    2^(-gap / ln 2) e (rms over N(0, 1) scores), i.e. 4.1e-4 of the output at 13
+    nats and less than that at 10; beside the rounding of the other
+    probabilities and of the output, 2.5e-4 (fp16) or 2e-3 (bf16). Bound: twice
+    the root of the sum of the squares."""
+    from delta_attention import ops
+    H, Hkv, D, N, n = 8, 2, 128, 12000, 64
+    q, k, v = gen_qkv(1, H, Hkv, N, D, seed=3, dtype=torch.float32)
+    q[..., 0] = 4.0
+    k[..., 0] = 0.0
+    k[:, :, 0] = 0.0
+    k[:, :, 0, 0] = gap * D ** 0.5 / 4.0
+    v[:, :, 0] = 0.0
+    q, k, v = (t.to(dtype) for t in (q, k, v))
+    rows = torch.arange(N - n, N, device="cuda")
+    out = ops.qsparse_attention(q, k, v, rows, D ** -0.5, q_rows=rows)
+    ref = O.qsparse_attention(np64(q)[:, :, N - n:], np64(k), np64(v), rows.cpu().numpy(), D ** -0.5)
+    err = np.linalg.norm(np64(out).ravel() - ref.ravel()) / np.linalg.norm(ref)
+    base = 2.5e-4 if dtype == torch.float16 else 2e-3
+    sub = 4.1e-4 if dtype == torch.float16 else 0.0
+    print(f"dominant first key {dtype} gap {gap}: rel {err:.3g}", flush=True)
+    assert err <= 2 * (base ** 2 + sub ** 2) ** 0.5, err
