@@ -44,10 +44,11 @@ struct AdaptArgs {
   int* log_n;
   // full_state: state holds 7 ints {gamma, n, n_recompute, slot0, step, have
   // rows ahead, rows ahead to compute now}, all written for the next chunk.
-  // spec_gamma > 0: the n_ahead dense rows at multiples of spec_gamma are
-  // computed in one launch, before chunk 0 (state[5] starts at 1) or behind the
-  // first of chunks 0 .. try_chunks - 1 whose decision leaves the next chunk a
-  // use for them (state[6] = n_ahead for that launch, else 0). With them, a
+  // spec_gamma > 0: the dense rows at multiples of spec_gamma are computed in
+  // one launch, before chunk 0 (state[5] starts at 1) or, from the next chunk's
+  // first row on, behind the first chunk with such a launch (n_ahead > 0: the
+  // rows it would compute) whose decision leaves the next chunk a use for them
+  // (state[6] = n_ahead for that launch, else 0). With them, a
   // chunk whose anchors are all such rows (stride and start multiples of
   // spec_gamma) reads them at slots slot0 + j * step and recomputes none; any
   // other chunk (every chunk with spec_gamma 0) has slot0 = -1 and recomputes
@@ -55,7 +56,7 @@ struct AdaptArgs {
   // sel_log[2 c .. 2 c + 1] logs this chunk's {slot0, step}.
   bool full_state;
   int spec_gamma;
-  int n_ahead, try_chunks;
+  int n_ahead;
   int* sel_log;
 };
 

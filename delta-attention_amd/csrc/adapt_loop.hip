@@ -15,10 +15,11 @@
 // multiple of gamma0 below s_p are computed ahead in one launch; a chunk whose
 // stride is a multiple of gamma0 (the starting stride and every doubling of it)
 // takes its anchors' rows from there, any other chunk recomputes its anchors.
-// The launch follows the first of the early chunks whose decision leaves the
-// next chunk such a stride (before chunk 0 in short layers): where the stride
-// falls at once and stays low the rows ahead would be wasted, 0.23 of 2.9 ms at
-// 40K tokens (2.95 -> 2.72 ms without them). Per chunk c:
+// The launch follows the first chunk whose decision leaves the next chunk such
+// a stride (see ahead_after; before chunk 0 in short layers) and covers the
+// rows from that chunk on: where the stride falls at once and stays low the
+// rows ahead would be wasted, 0.23 of 2.9 ms at 40K tokens (2.95 -> 2.72 ms
+// without them). Per chunk c:
 //   kernel (2) over the chunk's anchors when it recomputes them (a launch
 //     over a device-held row count that is zero otherwise), into one of two
 //     row buffers;
@@ -49,13 +50,29 @@ int delta_add_chunk(void* out, const int64_t o_str[3], const void* dense,
                     int max_n, int row_end, int s_p, int B, int H, int D, int n_grid, int dtype,
                     hipStream_t s);
 
+int qsparse_rows_of(int n_plan, const void* q, const void* k, const void* v,
+                    const int64_t* q_rows, int n, const int* n_dev, int B, int Hq, int Hkv,
+                    int Sq, int Skv, int D, const int64_t q_str[3], const int64_t k_str[3],
+                    const int64_t v_str[3], void* o, const int64_t o_str[3], float sm_scale,
+                    void* workspace, size_t workspace_bytes, int dtype, hipStream_t stream);
+
 namespace {
 
 // The rows ahead wait for a chunk to show that they will be used in layers of
 // at least AHEAD_LAZY_CHUNKS chunks (two chunks at 6001 tokens: 313 us with the
-// rows ahead first, 323 us waiting), behind one of the first AHEAD_TRIES
-// chunks' decisions (a launch over no rows costs each of them a few us).
-constexpr int AHEAD_LAZY_CHUNKS = 4, AHEAD_TRIES = 4;
+// rows ahead first, 323 us waiting).
+constexpr int AHEAD_LAZY_CHUNKS = 4;
+
+// Whether the rows ahead are launched behind chunk c's decision (over no rows
+// where that leaves no use for them, or they are there already): behind each
+// of the first chunks, then behind every fourth, so that a stride that comes
+// back late recomputes at most three more chunks. 128K tokens whose stride is
+// back at its start in chunk 7 / 11: 8.07 / 8.41 ms (8.87 / 9.16 behind the
+// first four chunks only, 7.97 / 8.49 with all rows computed before chunk 0);
+// a launch behind every chunk gave the same there and cost a layer that keeps
+// its stride 1.5 %.
+inline bool ahead_after(int c, int nc) { return c + 1 < nc && (c < 4 || c % 4 == 3); }
+
 constexpr int NEV = 4;      // events per ring; a ring slot is reused NEV chunks later
 
 // Rows per key-sparse launch on the second stream, in whole chunks of at least
@@ -256,8 +273,6 @@ extern "C" int da_adapt_layer_fwd(const void* q, const void* k, const void* v, v
   ad.log_mean = log_mean; ad.log_min = log_min; ad.log_gamma = log_gamma; ad.log_n = log_n;
   ad.full_state = true;
   ad.spec_gamma = use_ahead ? gamma0 : 0;
-  ad.n_ahead = p.n_ahead;
-  ad.try_chunks = lazy ? AHEAD_TRIES : 0;
   ad.sel_log = use_ahead ? sel_log : nullptr;
 
   // chunk c's recompute launch and its decision chain (the key-sparse rows
@@ -287,6 +302,9 @@ extern "C" int da_adapt_layer_fwd(const void* q, const void* k, const void* v, v
     else cs.a = dense;
     ad.chunk = c; ad.next_start = end; ad.next_end = next_end;
     ad.rows_next = next_end > end ? rows_c + max_n : nullptr;
+    // the slots of the rows ahead from the next chunk on
+    const int slot0 = lazy && ahead_after(c, p.nc) ? end / gamma0 : p.n_ahead;
+    ad.n_ahead = p.n_ahead - slot0;
     // the grids of the cosines and the broadcast are sized for a chunk at the
     // first stride and loop over more anchors (fewer empty workgroups; the
     // launches' time beside the key-sparse launches did not change)
@@ -298,10 +316,10 @@ extern "C" int da_adapt_layer_fwd(const void* q, const void* k, const void* v, v
         : delta_add_chunk(out, o_str, dense, dn_bhr, nullptr, nullptr, nullptr, rows_c,
                           log_n + c, max_n, end, s_p, B, Hq, D, p.n_live, dtype, st);
     // the rows ahead, if this chunk's decision turned them on
-    if (r == DA_OK && lazy && c < AHEAD_TRIES && c + 1 < p.nc)
-      r = da_qsparse_attn_fwd_live(q, k, v, ahead_rows, ahead_rows, 0, p.n_ahead, p.n_ahead,
-                                   state + 6, B, Hq, Hkv, S, s_p, D, q_str, k_str, v_str, ahead,
-                                   ah_bhr, sm_scale, ws_ahead, p.ws_ahead_bytes, dtype, st);
+    if (r == DA_OK && ad.n_ahead > 0)
+      r = qsparse_rows_of(p.n_ahead, q, k, v, ahead_rows + slot0, ad.n_ahead, state + 6, B, Hq,
+                          Hkv, S, s_p, D, q_str, k_str, v_str, (char*)ahead + (size_t)slot0 * D * 2,
+                          ah_bhr, sm_scale, ws_ahead, p.ws_ahead_bytes, dtype, st);
     return r;
   };
   const int per_launch =

@@ -188,7 +188,7 @@ __global__ __launch_bounds__(256) void adapt_next_kernel(AdaptArgs a) {
     if (a.full_state) {
       const bool fits = a.spec_gamma > 0 && g % a.spec_gamma == 0 &&
                         a.next_start % a.spec_gamma == 0;
-      const bool now = fits && !a.state[5] && a.chunk < a.try_chunks;
+      const bool now = fits && !a.state[5] && a.n_ahead > 0;
       if (now) a.state[5] = 1;
       a.state[6] = now ? a.n_ahead : 0;
       const bool ahead = fits && a.state[5];

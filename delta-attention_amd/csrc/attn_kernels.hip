@@ -1401,6 +1401,7 @@ struct QsparsePlan {
   int64_t vis;      // bound of a row tile's list
   bool f32;         // float partials
   bool grow;        // live launches: split length from the live row tiles
+  int lane_rows;    // rows that the merge's lanes are set for, where more than the launch's
 };
 
 // Rows per workgroup of a launch: for the head_dim-128 key-sparse launches
@@ -1431,6 +1432,7 @@ static QsparsePlan plan_qsparse(int B, int Hq, int Hkv, int n, int64_t vis, int 
   QsparsePlan p;
   p.f32 = f32;
   p.grow = false;
+  p.lane_rows = 0;
   const int G = Hq / Hkv;
   p.bm = bm;
   p.n_mtiles = (int)(((int64_t)n * G + bm - 1) / bm);
@@ -1509,14 +1511,8 @@ static size_t rows_ws_bytes(int B, int Hq, int Hkv, int n, int Skv, int D) {
   return p.n_items <= 0 || e.n_items <= 0 ? 0 : p.ws_bytes > e.ws_bytes ? p.ws_bytes : e.ws_bytes;
 }
 
-// Split plan for n rows of which about n_live hold keys (the others are -1
-// rows with empty tile lists: the adaptive stride's padded row lists): the
-// items per row tile follow the plan of n_live rows, the grid covers all n.
-static QsparsePlan plan_rows_live(int B, int Hq, int Hkv, int n, int n_live, int Skv, int D,
-                                  bool ends_seq) {
-  if (n_live >= n || n_live < 1) return plan_rows(B, Hq, Hkv, n, Skv, D, ends_seq);
-  QsparsePlan p = plan_rows(B, Hq, Hkv, n_live, Skv, D, false);
-  p.grow = true;
+// The items of `p`, planned for another row count, over n rows.
+static void cover_rows(QsparsePlan& p, int B, int Hq, int Hkv, int n, int D) {
   const int G = Hq / Hkv;
   p.n_mtiles = (int)(((int64_t)n * G + p.bm - 1) / p.bm);
   const int64_t base = (int64_t)B * Hkv * p.n_mtiles;
@@ -1525,6 +1521,17 @@ static QsparsePlan plan_rows_live(int B, int Hq, int Hkv, int n, int n_live, int
   p.n_items = fits ? (int)items : 0;
   p.ws_rows = (int)min((int64_t)p.bm, (int64_t)n * G);
   p.ws_bytes = fits ? (size_t)p.n_items * p.ws_rows * part_row_bytes(p, D) : 0;
+}
+
+// Split plan for n rows of which about n_live hold keys (the others are -1
+// rows with empty tile lists: the adaptive stride's padded row lists): the
+// items per row tile follow the plan of n_live rows, the grid covers all n.
+static QsparsePlan plan_rows_live(int B, int Hq, int Hkv, int n, int n_live, int Skv, int D,
+                                  bool ends_seq) {
+  if (n_live >= n || n_live < 1) return plan_rows(B, Hq, Hkv, n, Skv, D, ends_seq);
+  QsparsePlan p = plan_rows(B, Hq, Hkv, n_live, Skv, D, false);
+  p.grow = true;
+  cover_rows(p, B, Hq, Hkv, n, D);
   return p;
 }
 
@@ -1845,7 +1852,8 @@ static int run_qsparse(const QsparsePlan& p, const void* q, const void* k, const
   // lanes; workgroups per row tile cover its valid rows only
   {
     const int64_t rows = min((int64_t)p.bm, (int64_t)n * a.G);
-    const int64_t tasks = (int64_t)B * Hkv * p.n_mtiles * rows * (D / 8);
+    const int64_t all = (int64_t)max(p.lane_rows, n) * a.G;
+    const int64_t tasks = (int64_t)B * Hkv * ((all + p.bm - 1) / p.bm) * min((int64_t)p.bm, all) * (D / 8);
     m.lanes = 4;
     while (m.lanes < 16 && m.lanes * 4 < p.n_splits) m.lanes <<= 1;
     while (m.lanes > 1 && tasks * m.lanes > (1 << 18)) m.lanes >>= 1;
@@ -1895,7 +1903,7 @@ static int qsparse_fwd(const void* q, const void* k, const void* v,
                        int epi, int n_anchor, void* delta, const int64_t d_str[3],
                        float sm_scale, void* workspace, size_t workspace_bytes,
                        int dtype, void* stream, float* lse, int n_live,
-                       const int* n_rows_dev = nullptr) {
+                       const int* n_rows_dev = nullptr, int n_plan = 0) {
   int rc;
   if ((rc = check_common(B, Hq, Hkv, D, dtype)) != DA_OK) return rc;
   if (n < 0 || Sq < 0 || Skv < 0 || rl_bstride < 0 || n_live < 1) return DA_ERR_INVALID_ARG;
@@ -1914,7 +1922,12 @@ static int qsparse_fwd(const void* q, const void* k, const void* v,
       !strides8(q_str) || !strides8(k_str) || !strides8(v_str) || !strides8(o_str))
     return DA_ERR_ALIGNMENT;
   if (!kv_rows_ok(k_str, v_str)) return DA_ERR_INVALID_ARG;
-  const QsparsePlan p = plan_rows_live(B, Hq, Hkv, n, n_live, Skv, D, q_rows == nullptr);
+  QsparsePlan p = n_plan > n ? plan_rows(B, Hq, Hkv, n_plan, Skv, D, q_rows == nullptr)
+                             : plan_rows_live(B, Hq, Hkv, n, n_live, Skv, D, q_rows == nullptr);
+  if (n_plan > n) {
+    p.lane_rows = n_plan;
+    cover_rows(p, B, Hq, Hkv, n, D);
+  }
   return run_qsparse(p, q, k, v, q_rows, row_last, rl_bstride, n, B, Hq, Hkv, Sq, Skv, D,
                      q_str, k_str, v_str, o, o_str, epi, n_anchor, delta, d_str, 0, 0,
                      sm_scale, workspace, workspace_bytes, dtype, stream, nullptr, nullptr,
@@ -1933,6 +1946,23 @@ extern "C" int da_qsparse_attn_fwd(const void* q, const void* k, const void* v,
                      k_str, v_str, o, o_str, epi, n_anchor, delta, d_str, sm_scale, workspace,
                      workspace_bytes, dtype, stream, nullptr, 0x7fffffff);
 }
+
+namespace da {
+
+// Selected rows as da_qsparse_attn_fwd computes them among n_plan rows (the
+// same splits and order of summation, its workspace), n <= n_plan of them;
+// with n_dev, the first *n_dev of those.
+int qsparse_rows_of(int n_plan, const void* q, const void* k, const void* v,
+                    const int64_t* q_rows, int n, const int* n_dev, int B, int Hq, int Hkv,
+                    int Sq, int Skv, int D, const int64_t q_str[3], const int64_t k_str[3],
+                    const int64_t v_str[3], void* o, const int64_t o_str[3], float sm_scale,
+                    void* workspace, size_t workspace_bytes, int dtype, hipStream_t stream) {
+  return qsparse_fwd(q, k, v, q_rows, q_rows, 0, n, B, Hq, Hkv, Sq, Skv, D, q_str, k_str, v_str,
+                     o, o_str, DA_EPI_OUTPUT, 0, nullptr, nullptr, sm_scale, workspace,
+                     workspace_bytes, dtype, stream, nullptr, 0x7fffffff, n_dev, n_plan);
+}
+
+}  // namespace da
 
 extern "C" size_t da_qsparse_workspace_bytes_live(int B, int Hq, int Hkv, int n, int n_live, int Skv,
                                                   int D) {
