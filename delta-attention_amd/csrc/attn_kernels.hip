@@ -843,8 +843,9 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
     }
   }
 
-  // Two passes at most. Every row's reference max is its first visible tile's
-  // max; it moves only by more than THRESH. The first pass takes row maxima
+  // Two passes at most (head_dim 256: the exact one alone). Every row's
+  // reference max is its first visible tile's max; it moves only by more than
+  // THRESH. The first pass takes row maxima
   // only while a row lacks its reference (in the key-sparse modes with sinks,
   // the first tile sets every row's), which keeps the max reduction off the
   // per-tile path between the PV products and the barrier. A row whose max
@@ -930,13 +931,22 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
       step(t, Last(), exact_tag, sa, sb);
     }
   };
-  run(std::false_type());
-  // the barrier inside also orders the first pass's last LDS reads before
-  // the second pass refills the stages
-  bool big = false;
+  if constexpr (D > 128) {
+    // The exact pass alone at head_dim 256: with every tile's row max it takes
+    // 2-3 % longer where no max moves (509 rows of 16 heads against 16901 keys
+    // 141 -> 144 us, a layer of 8009 tokens 329 -> 338), while a first pass that
+    // is run again took 1.7 times as long as this one where they do (key norms
+    // growing 12-fold along the sequence: 253 -> 149 and 647 -> 392 us)
+    run(std::true_type());
+  } else {
+    run(std::false_type());
+    // the barrier inside also orders the first pass's last LDS reads before
+    // the second pass refills the stages
+    bool big = false;
 #pragma unroll
-  for (int rg = 0; rg < RG; ++rg) big = big || (valid[rg] && !(l_i[rg] <= 0.5f * LSUM));
-  if (__syncthreads_or(big)) run(std::true_type());
+    for (int rg = 0; rg < RG; ++rg) big = big || (valid[rg] && !(l_i[rg] <= 0.5f * LSUM));
+    if (__syncthreads_or(big)) run(std::true_type());
+  }
 
   // ---- epilogue ----
   if constexpr (AGPR_O) {

@@ -50,3 +50,31 @@ def test_exact_pass(gpu, kind, dtype):
     sp = ops.sparse_attention(q, k, v, window=256, sink=16, sm_scale=scale)
     assert_close(np64(sp), O.sparse_attention(np64(q), np64(k), np64(v), 256, 16, scale),
                  what=f"key-sparse d256 {kind} {dtype}")
+
+
+def test_moving_maxima_cost_no_second_pass(gpu):
+    """Keys whose norms grow 12x along the sequence move every row's reference
+    max. The tiles are still computed once: the launch takes at most 1.4 times
+    as long as on keys of one norm (two passes: 1.8 times; the smallest of
+    several batches of launches each)."""
+    from delta_attention.delta_kernel import attention
+    N, n, scale = 16901, 509, 256 ** -0.5
+    q, k, v = gen_qkv(1, 16, 4, n, 256, seed=7, N=N)
+    rows = torch.arange(N - n, N, device="cuda")[None]
+    grow = (k.float() * torch.linspace(1.0, 12.0, N, device="cuda")[None, None, :, None]).to(k.dtype)
+
+    def us(kk):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        best = float("inf")
+        for _ in range(6):
+            a.record()
+            for _ in range(20):
+                attention(q, kk, v, rows, scale)
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b) * 50)
+        return best
+
+    flat, moving = us(k), us(grow)
+    print(f"d256 rows: one norm {flat:.1f} us, growing {moving:.1f} us", flush=True)
+    assert moving <= 1.4 * flat, (flat, moving)
