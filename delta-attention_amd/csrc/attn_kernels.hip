@@ -1187,8 +1187,8 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
 
 // ---------------------------------------------------------------------------
 // Split-KV merge + epilogue of kernel (2). `wgs` workgroups per (b, kv head,
-// m tile) cover its valid rows x D/8 column chunks; each (row, chunk) task is
-// shared by P = `lanes` consecutive threads that take every P-th split and
+// m tile) cover its valid rows x column chunks (8 columns, or 4 in small merges
+// of float partials); each (row, chunk) task is shared by P = `lanes` consecutive threads that take every P-th split and
 // combine (max, sum, O) by xor-shuffles, so long split lists (decode rows)
 // are read with P loads in flight per task.
 struct MergeArgs {
@@ -1200,7 +1200,7 @@ struct MergeArgs {
   const int* n_kv_dev;   // as in AttnArgs
   const int* n_rows_dev; // as in AttnArgs: only the live row tiles are merged
   int window, sink;
-  int lanes;        // P: threads sharing one (row, 8-column) task, splits s = p mod P
+  int lanes;        // P: threads sharing one (row, column chunk) task, splits s = p mod P
   int wgs;          // workgroups per row tile
   int vis, slots;           // as in AttnArgs
   const void* part_o;       // O / l per split row (as in AttnArgs)
@@ -1220,11 +1220,13 @@ struct MergeArgs {
   float* lse;
 };
 
-// F32: the partials are floats (AttnArgs::part_f32).
-template <typename T, int D, bool F32>
+// F32: the partials are floats (AttnArgs::part_f32). CW: columns per task.
+template <typename T, int D, bool F32, int CW>
 __global__ __launch_bounds__(MTHR) void qsparse_merge_kernel(MergeArgs a) {
   using E = Elt<T>;
-  constexpr int CPR = D / 8;   // 8-column chunks per row
+  constexpr int CPR = D / CW;                   // column chunks per row
+  constexpr int NX = CW * (F32 ? 4 : 2) / 16;   // 16-byte pieces of a partial per task
+  typedef uint32_t Out __attribute__((ext_vector_type(CW / 2)));
   __shared__ int s_hmax[4], s_lmin[4];
   int tile = blockIdx.x / a.wgs;
   const int sub = blockIdx.x % a.wgs;
@@ -1294,19 +1296,18 @@ __global__ __launch_bounds__(MTHR) void qsparse_merge_kernel(MergeArgs a) {
     // a lane has all its partial reads in flight at once.
     constexpr int MU = 4;
     float M = NEG_BIG, L = 0.f;
-    float acc[8];
+    float acc[CW];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e] = 0.f;
-    auto take = [&](float m, float l, const float (&o)[8]) __attribute__((always_inline)) {
+    for (int e = 0; e < CW; ++e) acc[e] = 0.f;
+    auto take = [&](float m, float l, const float (&o)[CW]) __attribute__((always_inline)) {
       const float mn = fmaxf(M, m);
       const float wa = fast_exp2(M - mn), wb = fast_exp2(m - mn) * l;
       L = L * wa + wb;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) acc[e] = acc[e] * wa + o[e] * wb;
+      for (int e = 0; e < CW; ++e) acc[e] = acc[e] * wa + o[e] * wb;
       M = mn;
     };
     for (int s0 = p; s0 < nsv; s0 += MU * P) {
-      constexpr int NX = F32 ? 2 : 1;
       float ms[MU], ls[MU];
       u32x4 xs[MU][NX];
 #pragma unroll
@@ -1328,15 +1329,15 @@ __global__ __launch_bounds__(MTHR) void qsparse_merge_kernel(MergeArgs a) {
       }
 #pragma unroll
       for (int u = 0; u < MU; ++u) {
-        float o[8];
+        float o[CW];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
+        for (int e = 0; e < 4 * NX; ++e) {
+          const uint32_t x = xs[u][e / 4][e % 4];
           if constexpr (F32) {
-            o[e] = __uint_as_float(xs[u][0][e]);
-            o[4 + e] = __uint_as_float(xs[u][1][e]);
+            o[e] = __uint_as_float(x);
           } else {
-            o[2 * e] = E::lo(xs[u][0][e]);
-            o[2 * e + 1] = E::hi(xs[u][0][e]);
+            o[2 * e] = E::lo(x);
+            o[2 * e + 1] = E::hi(x);
           }
         }
         take(ms[u], ls[u], o);
@@ -1344,57 +1345,54 @@ __global__ __launch_bounds__(MTHR) void qsparse_merge_kernel(MergeArgs a) {
     }
     // the P lanes of the task combine their states the same way
     for (int off = 1; off < P; off <<= 1) {
-      float o[8];
+      float o[CW];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = __shfl_xor(acc[e], off);
+      for (int e = 0; e < CW; ++e) o[e] = __shfl_xor(acc[e], off);
       const float mo = __shfl_xor(M, off), lo = __shfl_xor(L, off);
       const float mn = fmaxf(M, mo);
       const float wa = fast_exp2(M - mn), wb = fast_exp2(mo - mn);
       L = L * wa + lo * wb;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) acc[e] = acc[e] * wa + o[e] * wb;
+      for (int e = 0; e < CW; ++e) acc[e] = acc[e] * wa + o[e] * wb;
       M = mn;
     }
     if (p != 0) return;
     const float inv = L > 0.f ? 1.f / L : 0.f;
+    Out pk;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e] *= inv;
+    for (int e = 0; e < CW / 2; ++e) pk[e] = E::pack2(acc[2 * e] * inv, acc[2 * e + 1] * inv);
 
     const int qrow = a.q_rows ? (int)min(max(a.q_rows[i], (int64_t)0), (int64_t)(a.n_q - 1)) : i;
     if (a.epi == DA_EPI_OUTPUT) {
       if (a.lse && c == 0)
         a.lse[((int64_t)b * a.Hkv * G + h) * a.n_rows + i] = L > 0.f ? M + __builtin_log2f(L) : INFINITY;
-      char* op = (char*)a.o + ((int64_t)b * a.os_b + (int64_t)h * a.os_h + (int64_t)i * a.os_s + 8 * c) * esz;
-      u32x4 pk = {E::pack2(acc[0], acc[1]), E::pack2(acc[2], acc[3]),
-                  E::pack2(acc[4], acc[5]), E::pack2(acc[6], acc[7])};
+      char* op = (char*)a.o + ((int64_t)b * a.os_b + (int64_t)h * a.os_h + (int64_t)i * a.os_s + CW * c) * esz;
       if (a.add) {
-        const u32x4 av = *(const u32x4*)((const char*)a.add +
-            ((int64_t)b * a.as_b + (int64_t)h * a.as_h + (int64_t)i * a.as_s + 8 * c) * esz);
+        const Out av = *(const Out*)((const char*)a.add +
+            ((int64_t)b * a.as_b + (int64_t)h * a.as_h + (int64_t)i * a.as_s + CW * c) * esz);
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+        for (int e = 0; e < CW / 2; ++e)
           pk[e] = E::pack2(E::lo(pk[e]) + E::lo(av[e]), E::hi(pk[e]) + E::hi(av[e]));
       }
-      *(u32x4*)op = pk;
+      *(Out*)op = pk;
     } else {
-      char* op = (char*)a.o + ((int64_t)b * a.os_b + (int64_t)h * a.os_h + (int64_t)qrow * a.os_s + 8 * c) * esz;
-      const u32x4 pk = {E::pack2(acc[0], acc[1]), E::pack2(acc[2], acc[3]),
-                        E::pack2(acc[4], acc[5]), E::pack2(acc[6], acc[7])};
+      char* op = (char*)a.o + ((int64_t)b * a.os_b + (int64_t)h * a.os_h + (int64_t)qrow * a.os_s + CW * c) * esz;
       if (a.epi == DA_EPI_DELTA && i < a.n_anchor) {
         // delta = rnd(rnd(dense) - sparse): the reference's bf16 subtraction.
-        const u32x4 sp = *(const u32x4*)op;
-        u32x4 dl;
+        const Out sp = *(const Out*)op;
+        Out dl;
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+        for (int e = 0; e < CW / 2; ++e)
           dl[e] = E::pack2(E::lo(pk[e]) - E::lo(sp[e]), E::hi(pk[e]) - E::hi(sp[e]));
         char* dp = (char*)a.delta +
-                   ((int64_t)b * a.ds_b + (int64_t)h * a.ds_h + (int64_t)i * a.ds_a + 8 * c) * esz;
-        *(u32x4*)dp = dl;
+                   ((int64_t)b * a.ds_b + (int64_t)h * a.ds_h + (int64_t)i * a.ds_a + CW * c) * esz;
+        *(Out*)dp = dl;
       } else if (a.epi == DA_EPI_DENSE && i < a.n_anchor) {
         char* dp = (char*)a.delta +
-                   ((int64_t)b * a.ds_b + (int64_t)h * a.ds_h + (int64_t)i * a.ds_a + 8 * c) * esz;
-        *(u32x4*)dp = pk;
+                   ((int64_t)b * a.ds_b + (int64_t)h * a.ds_h + (int64_t)i * a.ds_a + CW * c) * esz;
+        *(Out*)dp = pk;
       } else {
-        *(u32x4*)op = pk;
+        *(Out*)op = pk;
       }
     }
   }
@@ -1589,7 +1587,12 @@ static QsparsePlan plan_decode(int B, int Hq, int Hkv, int n_keys, int D, int wi
 // us (5.1 -> 6.0 TB/s; a plain read loop reaches 6.1 TB/s, 6.9 non-temporal),
 // 16 x 40 heads over 6007 keys 80 -> 71 us, 32 x 32 heads over 20000 keys 445
 // -> 400 us; where a repeated pass finds its keys in that cache (2 x 32 heads,
-// 20000 keys, 164 MB) non-temporal loads are slower, 35 -> 39 us.
+// 20000 keys, 164 MB) non-temporal loads are slower, 35 -> 39 us. With a device
+// key count the capacity decides: a model's other layers' caches pass through
+// that cache between two steps of one, so that fewer keys do not come from it
+// either (captured rows over the caches of 4-8 layers of 131072 slots: 20000
+// keys 25.4 -> 23.9 us a layer, 60000 keys 52.0 -> 48.1; 16 sequences of 3000 of
+// 8192 slots 45.8 -> 40.9; a single layer repeated alone is up to 4 % slower).
 static bool streams_kv(const QsparsePlan& p, int B, int Hkv, int D) {
   return p.n_mtiles == 1 && (int64_t)B * Hkv * p.vis * (BN * 4) * D > (int64_t)256 << 20;
 }
@@ -1624,9 +1627,10 @@ static void dispatch_attn(const AttnArgs& a, int D, int dtype, hipStream_t s) {
 }
 
 template <typename T, int D>
-static void launch_merge(const MergeArgs& m, int n_tiles, bool f32, hipStream_t s) {
-  if (f32) hipLaunchKernelGGL((qsparse_merge_kernel<T, D, true>), dim3(n_tiles), dim3(MTHR), 0, s, m);
-  else hipLaunchKernelGGL((qsparse_merge_kernel<T, D, false>), dim3(n_tiles), dim3(MTHR), 0, s, m);
+static void launch_merge(const MergeArgs& m, int n_tiles, bool f32, bool narrow, hipStream_t s) {
+  if (narrow) hipLaunchKernelGGL((qsparse_merge_kernel<T, D, true, 4>), dim3(n_tiles), dim3(MTHR), 0, s, m);
+  else if (f32) hipLaunchKernelGGL((qsparse_merge_kernel<T, D, true, 8>), dim3(n_tiles), dim3(MTHR), 0, s, m);
+  else hipLaunchKernelGGL((qsparse_merge_kernel<T, D, false, 8>), dim3(n_tiles), dim3(MTHR), 0, s, m);
 }
 
 // Query heads per key-sparse row tile: bm / 64 heads (64-row tiles) when
@@ -1859,7 +1863,12 @@ static int run_qsparse(const QsparsePlan& p, const void* q, const void* k, const
   // that many tasks already has enough loads in flight with one lane each,
   // and more lanes only add rounds of waves (128K layer: 36 us at one lane
   // vs 62 us at four; 32K: 11 vs 20 us), while a few decode rows need the
-  // lanes; workgroups per row tile cover its valid rows only
+  // lanes; workgroups per row tile cover its valid rows only. Few tasks over
+  // float partials (decode rows) take 4 columns each: one 16-byte load per
+  // split and task, twice the threads (captured decode rows, 32 heads: 2176 of
+  // 32771 keys 11.6 -> 11.2 us, 8000 keys 15.1 -> 14.4 us; 17 rows of 32 heads
+  // against 39339 keys, 2^17 threads already, 40.6 -> 41.1 us)
+  bool narrow;
   {
     const int64_t rows = min((int64_t)p.bm, (int64_t)n * a.G);
     const int64_t all = (int64_t)max(p.lane_rows, n) * a.G;
@@ -1867,7 +1876,8 @@ static int run_qsparse(const QsparsePlan& p, const void* q, const void* k, const
     m.lanes = 4;
     while (m.lanes < 16 && m.lanes * 4 < p.n_splits) m.lanes <<= 1;
     while (m.lanes > 1 && tasks * m.lanes > (1 << 18)) m.lanes >>= 1;
-    m.wgs = (int)((rows * (D / 8) * m.lanes + MTHR - 1) / MTHR);
+    narrow = p.f32 && tasks * m.lanes <= (1 << 14);
+    m.wgs = (int)((rows * (D / (narrow ? 4 : 8)) * m.lanes + MTHR - 1) / MTHR);
   }
   m.vis = a.vis; m.slots = a.slots;
   m.part_o = a.part_o; m.part_ml = a.part_ml; m.ws_rows = p.ws_rows; m.bm = p.bm;
@@ -1885,15 +1895,15 @@ static int run_qsparse(const QsparsePlan& p, const void* q, const void* k, const
   else dispatch_attn<MODE_QSPARSE>(a, D, dtype, s);
   const int n_tiles = B * Hkv * p.n_mtiles * m.wgs;
   if (dtype == DA_BF16) {
-    if (D == 128) launch_merge<__bf16, 128>(m, n_tiles, p.f32, s);
-    else if (D == 64) launch_merge<__bf16, 64>(m, n_tiles, p.f32, s);
-    else if (D == 256) launch_merge<__bf16, 256>(m, n_tiles, p.f32, s);
-    else launch_merge<__bf16, 32>(m, n_tiles, p.f32, s);
+    if (D == 128) launch_merge<__bf16, 128>(m, n_tiles, p.f32, narrow, s);
+    else if (D == 64) launch_merge<__bf16, 64>(m, n_tiles, p.f32, narrow, s);
+    else if (D == 256) launch_merge<__bf16, 256>(m, n_tiles, p.f32, narrow, s);
+    else launch_merge<__bf16, 32>(m, n_tiles, p.f32, narrow, s);
   } else {
-    if (D == 128) launch_merge<_Float16, 128>(m, n_tiles, p.f32, s);
-    else if (D == 64) launch_merge<_Float16, 64>(m, n_tiles, p.f32, s);
-    else if (D == 256) launch_merge<_Float16, 256>(m, n_tiles, p.f32, s);
-    else launch_merge<_Float16, 32>(m, n_tiles, p.f32, s);
+    if (D == 128) launch_merge<_Float16, 128>(m, n_tiles, p.f32, narrow, s);
+    else if (D == 64) launch_merge<_Float16, 64>(m, n_tiles, p.f32, narrow, s);
+    else if (D == 256) launch_merge<_Float16, 256>(m, n_tiles, p.f32, narrow, s);
+    else launch_merge<_Float16, 32>(m, n_tiles, p.f32, narrow, s);
   }
   return hipGetLastError() == hipSuccess ? DA_OK : DA_ERR_LAUNCH;
 }

@@ -11,7 +11,7 @@ from helpers import assert_close, np64
 pytestmark = pytest.mark.gpu
 
 
-def _case(B, H, Hkv, n, cap, D, dtype, dev_count):
+def _case(B, H, Hkv, n, cap, D, dtype, dev_count, add=False):
     from delta_attention import ops
     g = torch.Generator(device="cuda").manual_seed(n + D)
     q = torch.randn(B, 1, H, D, device="cuda", generator=g).to(dtype).transpose(1, 2)
@@ -20,7 +20,8 @@ def _case(B, H, Hkv, n, cap, D, dtype, dev_count):
     scale = D ** -0.5
     if dev_count:
         nk = torch.full((1,), n, dtype=torch.int32, device="cuda")
-        out = ops.decode_attention(q, k, v, window=0, sink=0, sm_scale=scale, n_keys=nk)
+        extra = torch.randn(B, H, 1, D, device="cuda", generator=g).to(dtype) if add else None
+        out = ops.decode_attention(q, k, v, window=0, sink=0, sm_scale=scale, n_keys=nk, add=extra)
     else:
         out = ops.decode_attention(q, k[:, :, :n], v[:, :, :n], window=0, sink=0, sm_scale=scale)
     G = H // Hkv
@@ -30,6 +31,8 @@ def _case(B, H, Hkv, n, cap, D, dtype, dev_count):
             kk, vv = k[b, h, :n].double().contiguous(), v[b, h, :n].double().contiguous()
             s = kk @ q[b, h * G:(h + 1) * G, 0].double().t().contiguous() * scale
             ref[b, h * G:(h + 1) * G, 0] = (torch.softmax(s, 0).t().contiguous() @ vv).cpu()
+    if add:
+        ref = ref + extra.double().cpu()
     assert_close(np64(out), ref.numpy(), what=f"decode B{B} H{H}/{Hkv} n{n} D{D} {dtype}")
 
 
@@ -45,3 +48,16 @@ def _case(B, H, Hkv, n, cap, D, dtype, dev_count):
 ])
 def test_decode_plan_edges(gpu, B, H, Hkv, n, cap, D, dtype, dev_count):
     _case(B, H, Hkv, n, cap, D, dtype, dev_count)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128, 256])
+@pytest.mark.parametrize("B,H,Hkv,n,dtype,add", [
+    (1, 8, 8, 700, torch.bfloat16, True),          # 16 threads a task, few tasks
+    (2, 32, 8, 5000, torch.float16, True),         # at head_dim 128 the most threads of the 4-column merge
+    (3, 32, 8, 5000, torch.bfloat16, False),       # past them
+    (4, 20, 4, 100, torch.float16, True),          # two splits
+])
+def test_merge_widths(gpu, B, H, Hkv, n, D, dtype, add):
+    """Both merge kernels over float partials (4 and 8 columns a task), with the
+    cached delta's add."""
+    _case(B, H, Hkv, n, n + 60, D, dtype, True, add)
