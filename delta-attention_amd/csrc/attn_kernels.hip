@@ -1139,23 +1139,36 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
     // long ones, a 16-byte row piece per lane after one permlane32 swap.
     // At half the fp32 volume, plain stores through L2 measured 0.5-1 %
     // faster than non-temporal ones; with fp32 partials the non-temporal form
-    // had kept the shared key/value chunk in L2 (split-kernel fetch 1.78 ->
-    // 1.59 GB).
+    // keeps the shared key/value chunk in L2 (64 rows of 32 heads that end 6000
+    // keys 25.3 -> 24.0 us, 150 of 8 heads x 2, head_dim 64, 20000 keys 35.3 ->
+    // 32.9; earlier fp32 partials: split-kernel fetch 1.78 -> 1.59 GB), but not
+    // for the few rows of a decode item (8000 keys 14.4 -> 14.6) nor beside the
+    // adaptive layer's other launches (selected rows: 11343 tokens 486 -> 490).
 #pragma unroll
     for (int rg = 0; rg < RG; ++rg) {
       if (!valid[rg]) continue;   // the merge reads the rows of the selection only
       const int r = (RG * wave + rg) * 32 + ln;
       if (a.part_f32) {
         float* po = (float*)a.part_o + ((int64_t)w * a.ws_rows + r) * D;
+        // every product first, so that the stores follow each other at once: the
+        // pieces of a row's cache lines then meet on their way out (with a
+        // product between two stores the non-temporal form lost 5-10 %)
+        f32x4 x[4 * NDT];
 #pragma unroll
-        for (int dt = 0; dt < NDT; ++dt)
+        for (int e = 0; e < 16 * NDT; ++e) x[e / 4][e % 4] = acc[rg][e / 16][e % 16] * inv[rg];
+        __builtin_amdgcn_sched_barrier(0);
+        f32x4* px = (f32x4*)(po + 4 * lg);
+        // (the empty statements keep the compiler from folding the two forms
+        // into one of plain stores)
+        if (!a.q_rows && a.ws_rows > 32) {
+          asm volatile("");
 #pragma unroll
-          for (int jq = 0; jq < 4; ++jq) {
-            f32x4 x;
+          for (int c = 0; c < 4 * NDT; ++c) __builtin_nontemporal_store(x[c], px + 2 * c);
+          asm volatile("");
+        } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) x[e] = acc[rg][dt][4 * jq + e] * inv[rg];
-            *(f32x4*)(po + 32 * dt + 8 * jq + 4 * lg) = x;
-          }
+          for (int c = 0; c < 4 * NDT; ++c) px[2 * c] = x[c];
+        }
       } else {
         uint32_t* po = (uint32_t*)a.part_o + ((int64_t)w * a.ws_rows + r) * (D / 2);
 #pragma unroll
@@ -1482,6 +1495,14 @@ static int64_t resident_slots(int D) { return 256 * attn_occupancy(D, 1); }
 // 40000 keys 208 -> 183 us). Their items hold at least sqrt(0.35 list) tiles:
 // a split costs the merge about a third of a key tile's time (40 rows of 32
 // heads at 8000 keys: 24.7 / 25.5 / 22.7 / 23.8 us at 4 / 5 / 8 / 10 tiles).
+// At head_dim 128 those rows take one item per CU in place of two where the two
+// would hold at most 16 tiles each, the shorter round stays at least 93 % full
+// and row tiles are at least half full: half the fp32 partials (25 rows of 32
+// / 4 heads x 2 against 16000 keys 37.1 -> 34.1 us, 64 of 32 / 8 heads at 20000
+// 40.5 -> 37.5, 100 of 40 at 12000 42.8 -> 41.5, 17 of 32 at 39339 40.5 -> 38.8,
+// though 40 of 32 at 30000 44.1 -> 45.4; longer items lose: 100 of 16 heads at
+// 50000, 25 tiles, 65.4 -> 67.1; 87 % full 48.8 -> 50.3; head_dim 64 29.9 -> 31.8;
+// row tiles a quarter full 42.4 -> 43.3).
 // Selected rows (q_rows) take at least 4 whatever the list, so that a row's
 // splits, and with them its bits, are the same in a launch over a prefix of
 // the keys (226 rows of 8 heads at 1531 keys 23.3 -> 14.5 us).
@@ -1504,6 +1525,12 @@ static QsparsePlan plan_rows(int B, int Hq, int Hkv, int n, int Skv, int D, bool
     if (chunk <= 80 || (ends_seq && chunk <= 160 && 20 * tiles * per_tile >= 19 * slots)) {
       int least = ends_seq ? 1 : 4;
       while (ends_seq && 20 * (int64_t)least * least < 7 * vis) ++least;
+      if (ends_seq && D == 128 && chunk <= 16 && tiles <= 256) {
+        const int64_t one = (vis + 256 / tiles - 1) / (256 / tiles);   // tiles of an item, one per CU
+        const bool full = tiles * ((vis + one - 1) / one) >= 238;
+        const bool half_rows = 2 * (int64_t)n * (Hq / Hkv) * B * Hkv >= bm * tiles;
+        if (full && half_rows && one > least) least = (int)one;
+      }
       return plan_qsparse(B, Hq, Hkv, n, vis, D, (int)(tiles * per_tile), least, bm, 0x7fffffff, true);
     }
   }

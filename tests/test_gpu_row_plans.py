@@ -42,6 +42,22 @@ def test_plan_edges(gpu, B, H, Hkv, n, N, D, selected):
         assert_close(np64(out[b:b + 1]), ref, what=f"B{B} n{n} N{N} D{D} batch {b}")
 
 
+@pytest.mark.parametrize("n,N", [
+    (64, 24000),      # row tiles just half full: one item per CU (31 of 12-13 tiles)
+    (63, 24000),      # less than half full: two (15-tile items)
+    (64, 65536),      # 16 tiles at two items per CU: one item of 32 tiles
+    (64, 65537),      # 17 tiles: two items
+])
+def test_ending_rows_per_cu(gpu, n, N):
+    """Rows that end a sequence around the rule for one or two items per CU."""
+    from delta_attention import ops
+    q, k, v = gen_qkv(1, 8, 8, n, 128, seed=N + n, N=N)
+    rows = torch.arange(N - n, N, device="cuda")
+    out = ops.qsparse_attention(q, k, v, rows[None], 128 ** -0.5)
+    ref = O.qsparse_attention(np64(q), np64(k), np64(v), rows.cpu().numpy(), 128 ** -0.5)
+    assert_close(np64(out), ref, what=f"n{n} N{N}")
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("gap", [10.0, 13.0])
 def test_dominant_first_key(gpu, dtype, gap):
