@@ -30,7 +30,8 @@
 // With a second stream, that stream takes the key-sparse pass over each
 // chunk's rows (kernel (1) over a row range) followed by the chunk's
 // recompute launch, then an event for `stream`; at the end it takes the dense
-// tail rows [s_p, S) scattered into out, and `stream` waits for it. The
+// tail rows [s_p, S) scattered into out (in short layers `stream` took them
+// before the last chunk's decision), and `stream` waits for it. The
 // recompute launch waits behind the key-sparse launch there, where its
 // workgroups (nearly always all of them empty) start in that launch's tail,
 // and not on `stream`, where they would wait for slots that the concurrent
@@ -322,6 +323,18 @@ extern "C" int da_adapt_layer_fwd(const void* q, const void* k, const void* v, v
                           ah_bhr, sm_scale, ws_ahead, p.ws_ahead_bytes, dtype, st);
     return r;
   };
+  auto tail_rows = [&](hipStream_t ts) -> int {
+    return da_qsparse_attn_fwd(q, k, v, tail, tail, 0, p.cut_n, B, Hq, Hkv, S, S, D, q_str, k_str,
+                               v_str, out, o_str, DA_EPI_SCATTER, 0, nullptr, nullptr, sm_scale,
+                               ws_tail, p.ws_tail_bytes, dtype, ts);
+  };
+  // Short layers: the dense tail goes to `stream` ahead of the last chunk's
+  // decision, under that chunk's key-sparse launch, instead of beside its
+  // cosines and broadcast, which waited for the tail's full round of
+  // workgroups (7125 tokens of 32 / 4 heads 392 -> 383 us, 11343 of 32 / 8 485 ->
+  // 477; 128K tokens 7.38 -> 7.42 ms, where the tail is long and the end of the
+  // layer hides under it)
+  const bool early_tail = side && p.nc > 0 && p.nc < AHEAD_LAZY_CHUNKS;
   const int per_launch =
       (int)std::max<int64_t>(1, ((int64_t)DA_ADAPT_SPARSE_ROWS + adapt_chunk - 1) / adapt_chunk);
   for (int c = 0; c < p.nc && rc == DA_OK; ++c) {
@@ -334,12 +347,10 @@ extern "C" int da_adapt_layer_fwd(const void* q, const void* k, const void* v, v
                                    side);
       if (rc != DA_OK) break;
     }
+    if (early_tail && c == p.nc - 1 && (rc = tail_rows(st)) != DA_OK) break;
     rc = chain(c);
   }
-  if (rc == DA_OK)
-    rc = da_qsparse_attn_fwd(q, k, v, tail, tail, 0, p.cut_n, B, Hq, Hkv, S, S, D, q_str, k_str,
-                             v_str, out, o_str, DA_EPI_SCATTER, 0, nullptr, nullptr, sm_scale,
-                             ws_tail, p.ws_tail_bytes, dtype, side ? side : st);
+  if (rc == DA_OK && !early_tail) rc = tail_rows(side ? side : st);
   if (side) {
     // whatever happened above, `stream` ends behind everything the second
     // stream was given
