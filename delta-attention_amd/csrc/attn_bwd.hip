@@ -86,7 +86,7 @@ struct BwdArgs {
   const int64_t* q_rows;         // selected rows: q row of list position i
   const int64_t* row_last;       // selected rows: last visible key, ascending
   int accumulate;                // outputs: out = rnd(out + rnd(grad))
-  int q32;                       // selected rows: every q row of a head within 32-bit byte offsets
+  int q32;                       // selected rows (dkdv_kernel): every q row of a head within 32-bit byte offsets
   void* q_gather;                // selected rows at head_dim 128: their q rows [B, Hq, n_rows, D]
   // dq kernel
   int n_mtiles, n_splits, chunk;
@@ -651,8 +651,9 @@ __global__ __launch_bounds__(NTHR, 1) void dkdv_kernel(BwdArgs a) {
       const int r = sigma32(ln);
       // Each MFMA pair's LDS fragments are read one pair ahead: at one wave
       // per SIMD nothing else hides a fragment read's latency, and read right
-      // before its MFMA every pair waited for it (backward 35.6 -> 31.8 ms at
-      // 128K keys; pinned by scheduling barriers it was slower, 37.7 ms)
+      // before its MFMA every pair waited for it (measured when head_dim 128
+      // still ran here: backward 35.6 -> 31.8 ms at 128K keys; pinned by
+      // scheduling barriers it was slower, 37.7 ms)
       {
         u32x4 qa[2], ga[2];
         qa[0] = read_rows<D>(qs, r, 0, lg);
@@ -922,7 +923,8 @@ __global__ __launch_bounds__(NTHR, 1) void dkdv_kernel(BwdArgs a) {
 // 4.59 -> 4.16 ms (this one about 2.73 -> 2.3); 8 / 8 heads at 16384 rows 858
 // -> 580 us. On copies that drop work: no DMA -350 us, no transposed reads
 // -190, no exponentials -150; what is left, 1.7 ms, is the MFMA issue rate of
-// one wave per SIMD (about 50 cycles each). Issued between the iterations
+// one wave per SIMD (24.5 ns each: 47 cycles at the 1.9 GHz that the power cap
+// leaves, 59 at 2.4; 32 at least). Issued between the iterations
 // instead of one a slot, the DMAs cost 160 us; plain row order instead of the
 // cyclic one 65 us.
 // ROWS: selected rows, list positions in place of rows: q comes from the
@@ -1677,8 +1679,9 @@ extern "C" int da_qsparse_attn_bwd(const void* q, const void* k, const void* v, 
                     dtype);
   if (rc != DA_OK) return rc;
   a.q_rows = q_rows; a.row_last = row_last;
-  // the dK/dV kernel's DMA addresses a head's gathered q rows from its row 0
-  // with 32-bit byte offsets (else it stages them through registers)
+  // at head_dim 32 and 64 the dK/dV kernel's DMA addresses a head's gathered q
+  // rows from its row 0 with 32-bit byte offsets, else it stages them through
+  // registers (head_dim 128 reads the gathered copy)
   a.q32 = (uint64_t)a.n_q * (uint64_t)a.qs_s * 2u <= 0xfffff000ull;
   a.window = 0; a.sink = 0; a.q_block = 1;
   const DqPlan dqp = plan_dq(B, Hkv, a.G, n, ((int64_t)Skv + DQ_BN - 1) / DQ_BN, true);

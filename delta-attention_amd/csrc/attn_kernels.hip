@@ -1503,9 +1503,10 @@ static int64_t resident_slots(int D) { return 256 * attn_occupancy(D, 1); }
 // though 40 of 32 at 30000 44.1 -> 45.4; longer items lose: 100 of 16 heads at
 // 50000, 25 tiles, 65.4 -> 67.1; 87 % full 48.8 -> 50.3; head_dim 64 29.9 -> 31.8;
 // row tiles a quarter full 42.4 -> 43.3).
-// Selected rows (q_rows) take at least 4 whatever the list, so that a row's
-// splits, and with them its bits, are the same in a launch over a prefix of
-// the keys (226 rows of 8 heads at 1531 keys 23.3 -> 14.5 us).
+// Selected rows (q_rows) take at least 4 whatever the list, so that while the
+// list is at most 4 tiles times the splits of a round a row's splits, and with
+// them its bits, are the same in a launch over a prefix of the keys (226 rows of
+// 8 heads at 1531 keys 23.3 -> 14.5 us); longer lists get longer items.
 //
 // Longer launches: ~8192 items (about half of them past the end of a causal
 // row tile's list), but at least 56 key tiles each: short items pay their
@@ -1884,8 +1885,9 @@ static int run_qsparse(const QsparsePlan& p, const void* q, const void* k, const
   m.B = B; m.n_rows_dev = n_rows_dev;
   m.window = window; m.sink = sink;
   // P threads per (row, column chunk) task: about 4 splits each, 4 to 16
-  // (at least 4 however few splits the plan has: a row's order of summation
-  // then depends on its own list, not on the keys the launch was planned for),
+  // (at least 4 however few splits the plan has: up to 16 of them, and as long
+  // as the tasks do not lower the count, a row's order of summation depends on
+  // its own list and not on the keys the launch was planned for),
   // but no more threads than about half the GPU holds (2^18): a merge with
   // that many tasks already has enough loads in flight with one lane each,
   // and more lanes only add rounds of waves (128K layer: 36 us at one lane

@@ -1,7 +1,6 @@
 """head_dim 256 at the edges of its tile loop: one to five 64-key tiles with
 and without a remainder, single rows and row counts around a 128-row tile, and
-inputs that send workgroups through the exact second pass, against the
-oracle's softmax (tolerance: the layer's parity bar, helpers.assert_close)."""
+inputs whose reference maxima move, against the oracle's softmax (tolerance: the layer's parity bar, helpers.assert_close)."""
 
 import numpy as np
 import pytest
@@ -29,8 +28,8 @@ def test_rows(gpu, n, N, dtype):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_exact_pass(gpu, kind, dtype):
     """Key norms growing 12x along the sequence, or 1 % of the keys at 40x:
-    rows whose reference max moves take the second pass, and every row keeps
-    the same bits whichever rows share its workgroup."""
+    every row keeps the same bits whichever rows share its workgroup, also where
+    their reference maxima move."""
     from delta_attention import ops
     from delta_attention.delta_kernel import attention
     from delta_attention.llama import repeat_kv

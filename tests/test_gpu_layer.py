@@ -287,11 +287,14 @@ def _with_heads(cases, H=8, Hkv=2, D=128):
 def test_adaptive_layer_composition_is_exact(gpu, B, s, chunk, gamma0, gmin, dtype, H, Hkv, D):
     """The one-call adaptive layer (da_adapt_layer_fwd) against the same
     steps issued one by one: the key-sparse pass over all rows; each chunk's
-    dense anchor rows from the same kernel (2) launch as inside, i.e. when
-    gamma0 divides adapt_chunk and the chunk's stride is a multiple of gamma0
-    the rows-ahead launch (every multiple of gamma0 below s_p, keys < s_p),
-    else the chunk's own launch (its -1-padded row list, keys < the chunk's
-    end, the same live-row plan); the deltas rnd(dense - sparse[anchor]) and
+    dense anchor rows, when gamma0 divides adapt_chunk and the chunk's stride
+    is a multiple of gamma0, from a launch over every multiple of gamma0 below
+    s_p (keys < s_p), else from the chunk's own launch (its -1-padded row list,
+    keys < the chunk's end, the same live-row plan). Inside, a chunk of a layer
+    of four and more recomputes its anchors until a launch of such rows exists;
+    at these sizes both launches cut their lists into 4-tile items and sum them
+    alike, so the rows have the same bits (where they do not:
+    test_gpu_adaptive_ahead.py); the deltas rnd(dense - sparse[anchor]) and
     rows rnd(sparse + delta) in torch bf16 ops (stride.py:26-40); and the dense
     tail. Bit-identical: the row selection, the per-chunk in-place broadcast,
     the row ranges of the sparse pass and the tail scatter change no bits."""
