@@ -843,8 +843,8 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
     }
   }
 
-  // Two passes at most (head_dim 256: the exact one alone). Every row's
-  // reference max is its first visible tile's max; it moves only by more than
+  // Two passes at most (key-sparse at head_dim 256: the exact one alone). Every
+  // row's reference max is its first visible tile's max; it moves only by more than
   // THRESH. The first pass takes row maxima
   // only while a row lacks its reference (in the key-sparse modes with sinks,
   // the first tile sets every row's), which keeps the max reduction off the
@@ -931,12 +931,13 @@ __global__ __launch_bounds__(NTHR, attn_occupancy(D, RG)) void attn_fwd_kernel(A
       step(t, Last(), exact_tag, sa, sb);
     }
   };
-  if constexpr (D > 128) {
-    // The exact pass alone at head_dim 256: with every tile's row max it takes
-    // 2-3 % longer where no max moves (509 rows of 16 heads against 16901 keys
-    // 141 -> 144 us, a layer of 8009 tokens 329 -> 338), while a first pass that
-    // is run again took 1.7 times as long as this one where they do (key norms
-    // growing 12-fold along the sequence: 253 -> 149 and 647 -> 392 us)
+  if constexpr (D > 128 && KSPARSE) {
+    // The exact pass alone: with every tile's row max it takes 2 % longer where
+    // no max moves (8009 rows of 16 heads 259 -> 265 us), while two passes took
+    // longer than the compiler-scheduled loop's one where they do (key norms
+    // growing 12-fold along the sequence: 532 us, 402 in that loop, 316 so). The
+    // row launches gained more from the schedule and keep two (509 rows against
+    // 16901 keys 139 us, 251 with growing keys, 318 before).
     run(std::true_type());
   } else {
     run(std::false_type());
